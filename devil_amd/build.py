@@ -21,7 +21,7 @@ LIB = os.path.join(HERE, "libdevil_hip.so")
 ROOT = os.path.dirname(HERE)
 
 SOURCES = ["kernels_epilogue.hip", "kernels_tile.hip", "kernels_mle.hip", "kernels_post.hip",
-           "kernels_design.hip", "kernels_prep.hip", "kernels_newod.hip",
+           "kernels_design.hip", "kernels_prep.hip", "kernels_newod.hip", "kernels_gene.hip",
            "devil_hip.cpp"]
 
 COMMON = [

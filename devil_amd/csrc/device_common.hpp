@@ -18,6 +18,13 @@ __device__ __forceinline__ int wave_index() {
   return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 }
 
+// v as a wave-uniform (scalar register) value; every lane holds the same.
+__device__ __forceinline__ double uniform_f64(double v) {
+  const int lo = __builtin_amdgcn_readfirstlane(__double2loint(v));
+  const int hi = __builtin_amdgcn_readfirstlane(__double2hiint(v));
+  return __hiloint2double(hi, lo);
+}
+
 __device__ __forceinline__ double wave_sum(double v) {
 #pragma unroll
   for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o, kWave);

@@ -676,6 +676,8 @@ void shape_design(const ColPlan& cp, int64_t n, int p, int cells_per_block, dv::
 struct TileHost {
   dv::TileDesign td{};   // FP64 design (16-cell blocks, packed columns)
   dv::TileDesign tdm{};  // mixed design (td for FP32, 32-cell steps for bf16)
+  const double* X = nullptr;    // device n x p design, column-major
+  const double* off = nullptr;  // device offsets
   int mixed = kMixedNone;
   DevBuf spec, specm, Xp, offp, eop, Kp, Xf, offf, Kf, xab, offl, kg, kh, kh2;
 };
@@ -685,6 +687,8 @@ int make_tile(devil_ctx* ctx, const double* Xd, const double* offd, const double
               int64_t n, int p, int mixed, TileHost& th, int64_t chunk_cells = 2048) {
   hipStream_t s = ctx->stream;
   th.mixed = mixed;
+  th.X = Xd;
+  th.off = offd;
   ColPlan cp;
   int rc;
   if ((rc = plan_columns(ctx, Xd, n, p, false, cp))) return rc;
@@ -1222,6 +1226,60 @@ int driver_rounds(devil_ctx* ctx, const dv::TileDesign& tfull, size_t part_cap, 
   return DEVIL_OK;
 }
 
+// The FP64 IRLS takes one workgroup per gene where the design stays in an
+// XCD's L2 (4 MB, shared with the counts of 32 CUs' genes).
+constexpr int64_t kGeneDesignBytes = (int64_t)2 << 20;
+
+bool gene_path(const TileHost& tl, int p) {
+  return (int64_t)sizeof(double) * (p + 1) * tl.td.n <= kGeneDesignBytes;
+}
+
+dv::GeneDesign gene_design(const TileHost& tl, int p) {
+  dv::GeneDesign gd{};
+  gd.n = tl.td.n;
+  gd.X = tl.X;
+  gd.off = tl.off;
+  std::memcpy(gd.kidx_pair, tl.td.kidx_pair, sizeof(gd.kidx_pair));
+  std::memcpy(gd.kidx_lin, tl.td.kidx_lin, sizeof(gd.kidx_lin));
+  std::memcpy(gd.ksum, tl.td.ksum, sizeof(gd.ksum));
+  // x_0 x_b == x_b for every b makes x_0 one or zero where it matters; summing
+  // to n, it is one everywhere
+  const int c0 = tl.td.kidx_lin[0];
+  gd.intercept = c0 >= 0 && tl.td.ksum[c0] == (double)tl.td.n;
+  for (int b = 0; b < p; ++b)
+    if (tl.td.kidx_pair[b] != tl.td.kidx_lin[b]) gd.intercept = 0;
+  return gd;
+}
+
+// One launch of the gene kernel over list[0 .. ngenes) (all genes [0, ngenes)
+// when list is null), with its launch record.
+int run_irls_gene(devil_ctx* ctx, const TileHost& tl, dv::Counts c, int p, const int32_t* list,
+                  int ngenes, double* beta, const double* kvec, int max_iter, double eps,
+                  int32_t* iters, int32_t* status) {
+  hipStream_t s = ctx->stream;
+  const size_t nrec = ctx->launches.size();
+  {
+    LaunchTimer lt(ctx, DEVIL_KERNEL_IRLS_FP64, 0.0);
+    DV_HIP(dv::launch_irls_gene(s, gene_design(tl, p), c, p, list, ngenes, beta, kvec, max_iter,
+                                eps, iters, status));
+  }
+  if (ctx->launches.size() > nrec) {  // timing: the bytes follow from the iterations
+    std::vector<int32_t> lh(list ? ngenes : 0);
+    if (list)
+      DV_HIP(hipMemcpyAsync(lh.data(), list, sizeof(int32_t) * ngenes, hipMemcpyDeviceToHost, s));
+    DV_HIP(hipStreamSynchronize(s));
+    const int last = list ? *std::max_element(lh.begin(), lh.end()) + 1 : ngenes;
+    std::vector<int32_t> ih(last);
+    DV_HIP(hipMemcpyAsync(ih.data(), iters, sizeof(int32_t) * last, hipMemcpyDeviceToHost, s));
+    DV_HIP(hipStreamSynchronize(s));
+    double sum = 0.0;
+    for (int i = 0; i < ngenes; ++i) sum += ih[list ? lh[i] : i];
+    ctx->launches[nrec].bytes = (double)count_elem_size(c.dtype) * (double)tl.td.n * sum;
+    collect_launches(ctx);
+  }
+  return DEVIL_OK;
+}
+
 int run_irls_tiled(devil_ctx* ctx, const TileHost& tl, dv::Counts c, int64_t G, int p,
                    double* beta, const double* kvec, int max_iter, double eps,
                    int32_t* iters, int32_t* status) {
@@ -1235,6 +1293,9 @@ int run_irls_tiled(devil_ctx* ctx, const TileHost& tl, dv::Counts c, int64_t G, 
     if (max_iter <= 0) DV_HIP(dv::launch_fill_i32(s, status, G, DEVIL_GENE_MAXITER));
     return DEVIL_OK;
   }
+  if (!mixed && gene_path(tl, p))
+    return run_irls_gene(ctx, tl, c, p, nullptr, (int)G, beta, kvec, max_iter, eps, iters,
+                         status);
   DevBuf act0, act1, cnt, part, rep, beta0;
   DV_ALLOC(act0, sizeof(int32_t) * G);
   DV_ALLOC(act1, sizeof(int32_t) * G);
@@ -1273,10 +1334,14 @@ int run_irls_tiled(devil_ctx* ctx, const TileHost& tl, dv::Counts c, int64_t G, 
     // FP64 refit of the replay genes from their starting beta
     DV_HIP(dv::launch_restart_genes(s, rep.as<int32_t>(), nr, p, beta0.as<double>(), beta,
                                     iters, status, bprev.as<double>()));
-    if ((rc = irls_rounds(ctx, tl, false, c, p, beta, kvec, max_iter, eps, iters, status,
-                          rep.as<int32_t>(), act1.as<int32_t>(), nrep, c0 + 3, nr,
-                          part.as<double>(), part_cap, nullptr, nullptr)))
-      return rc;
+    if (gene_path(tl, p))
+      rc = run_irls_gene(ctx, tl, c, p, rep.as<int32_t>(), nr, beta, kvec, max_iter, eps, iters,
+                         status);
+    else
+      rc = irls_rounds(ctx, tl, false, c, p, beta, kvec, max_iter, eps, iters, status,
+                       rep.as<int32_t>(), act1.as<int32_t>(), nrep, c0 + 3, nr,
+                       part.as<double>(), part_cap, nullptr, nullptr);
+    if (rc) return rc;
   }
   // The mixed trajectory leaves ~5e-7 absolute on beta; where a coefficient
   // is small that is a large relative error.  Such genes get their last step

@@ -196,6 +196,22 @@ hipError_t launch_polish_select(hipStream_t s, int64_t G, int p, const double* b
                                 int32_t* list, int32_t* nlist);
 hipError_t launch_iota(hipStream_t s, int32_t* p, int n);
 
+// IRLS of ngenes genes (list[0 .. ngenes), or all when list is null), one
+// workgroup per gene for all its iterations (kernels_gene.hip).  beta holds
+// the starting values; iters and status are written.  max_iter >= 1.
+struct GeneDesign {
+  int64_t n;
+  const double* X;    // n x p column-major
+  const double* off;  // n
+  int intercept;      // column 0 of X is all ones
+  int kidx_pair[55];  // as TileDesign's
+  int kidx_lin[10];
+  double ksum[DEVIL_NCP_MAX];
+};
+hipError_t launch_irls_gene(hipStream_t s, const GeneDesign& gd, Counts c, int p,
+                            const int32_t* list, int ngenes, double* beta, const double* kvec,
+                            int max_iter, double eps, int32_t* iters, int32_t* status);
+
 // One problem's share of a joint round (kernels_tile.hip): its round shape,
 // counts, active list and outputs, its workgroups of the accumulate grid and
 // its blocks of the update grid.
