@@ -1258,10 +1258,12 @@ int run_irls_gene(devil_ctx* ctx, const TileHost& tl, dv::Counts c, int p, const
                   int32_t* iters, int32_t* status) {
   hipStream_t s = ctx->stream;
   const size_t nrec = ctx->launches.size();
+  DevBuf next;
+  DV_ALLOC(next, sizeof(int32_t));
   {
     LaunchTimer lt(ctx, DEVIL_KERNEL_IRLS_FP64, 0.0);
-    DV_HIP(dv::launch_irls_gene(s, gene_design(tl, p), c, p, list, ngenes, beta, kvec, max_iter,
-                                eps, iters, status));
+    DV_HIP(dv::launch_irls_gene(s, gene_design(tl, p), c, p, list, ngenes, next.as<int32_t>(),
+                                beta, kvec, max_iter, eps, iters, status));
   }
   if (ctx->launches.size() > nrec) {  // timing: the bytes follow from the iterations
     std::vector<int32_t> lh(list ? ngenes : 0);

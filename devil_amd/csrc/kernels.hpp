@@ -198,7 +198,8 @@ hipError_t launch_iota(hipStream_t s, int32_t* p, int n);
 
 // IRLS of ngenes genes (list[0 .. ngenes), or all when list is null), one
 // workgroup per gene for all its iterations (kernels_gene.hip).  beta holds
-// the starting values; iters and status are written.  max_iter >= 1.
+// the starting values; iters and status are written.  max_iter >= 1.  next: a
+// device counter the launch uses.
 struct GeneDesign {
   int64_t n;
   const double* X;    // n x p column-major
@@ -209,8 +210,9 @@ struct GeneDesign {
   double ksum[DEVIL_NCP_MAX];
 };
 hipError_t launch_irls_gene(hipStream_t s, const GeneDesign& gd, Counts c, int p,
-                            const int32_t* list, int ngenes, double* beta, const double* kvec,
-                            int max_iter, double eps, int32_t* iters, int32_t* status);
+                            const int32_t* list, int ngenes, int32_t* next, double* beta,
+                            const double* kvec, int max_iter, double eps, int32_t* iters,
+                            int32_t* status);
 
 // One problem's share of a joint round (kernels_tile.hip): its round shape,
 // counts, active list and outputs, its workgroups of the accumulate grid and
