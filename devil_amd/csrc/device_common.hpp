@@ -305,14 +305,14 @@ __device__ inline double nb_f(double x) {
 }
 
 // Stirling remainder of lgamma for x >= 10.
-__device__ inline double lgamma_corr(double x) {
+__host__ __device__ inline double lgamma_corr(double x) {
   const double f = 1.0 / (x * x);
   return (1.0 / 12 - f * (1.0 / 360 - f * (1.0 / 1260 - f * (1.0 / 1680 -
           f * (1.0 / 1188 - f * (691.0 / 360360 - f * (1.0 / 156))))))) / x;
 }
 
 // log B(a, b) with the large-argument forms that avoid cancellation.
-__device__ inline double lbeta(double a, double b) {
+__host__ __device__ inline double lbeta(double a, double b) {
   const double p = fmin(a, b), q = fmax(a, b);
   const double half_log_2pi = 0.91893853320467274178;
   if (p >= 10.0) {
@@ -326,29 +326,42 @@ __device__ inline double lbeta(double a, double b) {
   return lgamma(p) + lgamma(q) - lgamma(p + q);
 }
 
-// Continued fraction of the regularised incomplete beta (modified Lentz).
+// 1/d from v_rcp_f64 refined by two Newton steps (about 1 ulp).
+__device__ __forceinline__ double rcp_f64(double d) {
+  double r = __builtin_amdgcn_rcp(d);
+  double e = fma(-d, r, 1.0);
+  r = fma(r, e, r);
+  e = fma(-d, r, 1.0);
+  return fma(r, e, r);
+}
+
+// Continued fraction of the regularised incomplete beta (modified Lentz).  It
+// stops where a factor is within two ulps of 1: with fused multiply-adds the
+// factors of a converged fraction keep moving by an ulp, and waiting for 1
+// itself took some lanes hundreds of further steps (a test of 20000 genes took
+// 245 us at 500 cells and 1550 us at 500000).
 __device__ inline double betacf(double a, double b, double x) {
-  const double tiny = 1e-300, epsr = 1e-16;
+  const double tiny = 1e-300, epsr = 4.5e-16;
   const double qab = a + b, qap = a + 1.0, qam = a - 1.0;
-  double c = 1.0, d = 1.0 - qab * x / qap;
+  double c = 1.0, d = 1.0 - qab * x * rcp_f64(qap);
   if (fabs(d) < tiny) d = tiny;
-  d = 1.0 / d;
+  d = rcp_f64(d);
   double h = d;
   for (int m = 1; m <= 100000; ++m) {
     const double m2 = 2.0 * m;
-    double aa = m * (b - m) * x / ((qam + m2) * (a + m2));
+    double aa = m * (b - m) * x * rcp_f64((qam + m2) * (a + m2));
     d = 1.0 + aa * d;
     if (fabs(d) < tiny) d = tiny;
-    c = 1.0 + aa / c;
+    c = 1.0 + aa * rcp_f64(c);
     if (fabs(c) < tiny) c = tiny;
-    d = 1.0 / d;
+    d = rcp_f64(d);
     h *= d * c;
-    aa = -(a + m) * (qab + m) * x / ((a + m2) * (qap + m2));
+    aa = -(a + m) * (qab + m) * x * rcp_f64((a + m2) * (qap + m2));
     d = 1.0 + aa * d;
     if (fabs(d) < tiny) d = tiny;
-    c = 1.0 + aa / c;
+    c = 1.0 + aa * rcp_f64(c);
     if (fabs(c) < tiny) c = tiny;
-    d = 1.0 / d;
+    d = rcp_f64(d);
     const double del = d * c;
     h *= del;
     if (fabs(del - 1.0) < epsr) break;
@@ -357,8 +370,9 @@ __device__ inline double betacf(double a, double b, double x) {
 }
 
 // log of 2*P(T_df > |t|) = log I_{df/(df+t^2)}(df/2, 1/2); exact in log space
-// where the probability underflows.
-__device__ inline double log_pt2_upper(double t, double df) {
+// where the probability underflows.  lb = lbeta(df/2, 1/2), the same for every
+// gene.
+__device__ inline double log_pt2_upper(double t, double df, double lb) {
   if (isnan(t) || isnan(df) || !(df > 0.0)) return __builtin_nan("");
   t = fabs(t);
   if (isinf(t)) return -__builtin_huge_val();
@@ -368,10 +382,12 @@ __device__ inline double log_pt2_upper(double t, double df) {
   const double lx = ldf - l_sum, lomx = 2.0 * lt - l_sum;
   const double x = exp(lx), omx = exp(lomx);
   const double a = 0.5 * df, b = 0.5;
-  const double lfront = a * lx + b * lomx - lbeta(a, b);
-  if (x < (a + 1.0) / (a + b + 2.0)) return lfront + log(betacf(a, b, x)) - log(a);
-  const double lc = lfront + log(betacf(b, a, omx)) - log(b);
-  return log1p(-exp(lc));
+  const double lfront = a * lx + b * lomx - lb;
+  // one fraction for both tails, so that a wave whose lanes differ runs it once
+  const bool low = x < (a + 1.0) / (a + b + 2.0);
+  const double fa = low ? a : b;
+  const double lc = lfront + log(betacf(fa, low ? b : a, low ? x : omx)) - log(fa);
+  return low ? lc : log1p(-exp(lc));
 }
 
 // ---------------------------------------------------------------------------
@@ -407,15 +423,6 @@ __device__ __forceinline__ double exp_f64(double x) {
   p = fma(p, r, 1.0);
   p = fma(p, r, 1.0);
   return ldexp(p, (int)n);
-}
-
-// 1/d from v_rcp_f64 refined by two Newton steps (about 1 ulp).
-__device__ __forceinline__ double rcp_f64(double d) {
-  double r = __builtin_amdgcn_rcp(d);
-  double e = fma(-d, r, 1.0);
-  r = fma(r, e, r);
-  e = fma(-d, r, 1.0);
-  return fma(r, e, r);
 }
 
 // 1/d from v_rcp_f64 (relative error below 4.6e-8 on gfx950, measured) and

@@ -29,7 +29,7 @@ __global__ void k_k_from_alpha(const double* __restrict__ alpha0, int64_t G,
 // ---------------------------------------------------------------------------
 __global__ void k_test_de(const double* __restrict__ beta, const double* __restrict__ bread,
                           const double* __restrict__ sandwich, int64_t G, int p, double df,
-                          const double* __restrict__ contrast, double max_lfc,
+                          double lb, const double* __restrict__ contrast, double max_lfc,
                           double* __restrict__ pval, double* __restrict__ logp,
                           double* __restrict__ lfc) {
   const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -40,13 +40,13 @@ __global__ void k_test_de(const double* __restrict__ beta, const double* __restr
   double v0 = 0.0;
   for (int a = 0; a < p; ++a)
     for (int bb = 0; bb < p; ++bb) v0 += contrast[a] * H[a + bb * p] * contrast[bb];
-  double lp = log_pt2_upper(fabs(l) / sqrt(v0), df);
+  double lp = log_pt2_upper(fabs(l) / sqrt(v0), df, lb);
   if (sandwich) {
     const double* S = sandwich + g * p * p;
     double v1 = 0.0;
     for (int a = 0; a < p; ++a)
       for (int bb = 0; bb < p; ++bb) v1 += contrast[a] * S[a + bb * p] * contrast[bb];
-    const double lp1 = log_pt2_upper(fabs(l) / sqrt(v1), df);
+    const double lp1 = log_pt2_upper(fabs(l) / sqrt(v1), df, lb);
     if (isnan(lp) || isnan(lp1)) lp = __builtin_nan("");
     else if (lp1 > lp) lp = lp1;
   }
@@ -357,7 +357,8 @@ hipError_t launch_test_de(hipStream_t s, const double* beta, const double* bread
                           double* adj) {
   if (G <= 0) return hipSuccess;
   const dim3 g1((unsigned)((G + 255) / 256));
-  hipLaunchKernelGGL(k_test_de, g1, dim3(256), 0, s, beta, bread, sandwich, G, p, df,
+  const double lb = df > 0.0 ? lbeta(0.5 * df, 0.5) : 0.0;
+  hipLaunchKernelGGL(k_test_de, g1, dim3(256), 0, s, beta, bread, sandwich, G, p, df, lb,
                      contrast, max_lfc, pval, logp, lfc);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
