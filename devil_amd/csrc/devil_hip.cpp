@@ -808,9 +808,17 @@ int tile_from_device(devil_ctx* ctx, const double* X, const double* offset, int6
   return DEVIL_OK;
 }
 
-// Chunk table of the post-IRLS passes: cell ranges of at most about
+// Chunk table of the init and post-IRLS passes: cell ranges of at most about
 // max(2048, n / 64) cells, never straddling a patient block; the count is
-// rounded up to a multiple of 8 with empty chunks (one XCD per chunk).
+// rounded up to a multiple of 8 with empty chunks (one XCD per chunk).  With
+// few genes the ranges are shorter, so that the passes' waves (a 16-gene tile
+// and a range each) fill the GPU: kPostWaves of them, down to 128 cells and
+// up to 256 ranges.  64 genes x 2000 cells ran on 4 waves of 125 blocks each,
+// 97 us for the init pass and 109 us for the bread; 64 waves take 11 and
+// 10 us.  genes = 0 keeps the long ranges: the mixed clustered pass sums the
+// pair columns in FP32 over a range, so its ranges set its rounding.
+constexpr int64_t kPostWaves = 4096;
+
 struct ChunkHost {
   std::vector<int64_t> c0, c1;
   std::vector<int32_t> cl;
@@ -818,17 +826,34 @@ struct ChunkHost {
   dv::ChunkTable ct{};
 };
 
-int build_chunks(devil_ctx* ctx, int64_t n, const int32_t* ends, int C, ChunkHost& ch) {
-  const int64_t target = std::max<int64_t>(2048, (n + 63) / 64);
+int build_chunks(devil_ctx* ctx, int64_t n, const int32_t* ends, int C, int64_t genes,
+                 ChunkHost& ch) {
+  int64_t target = std::max<int64_t>(2048, (n + 63) / 64);
+  bool fine = false;
+  if (genes > 0) {
+    const int64_t want = (kPostWaves * 16 + genes - 1) / genes;  // ranges
+    const int64_t cells = 16 * ((n / want + 15) / 16);
+    const int64_t least = std::max<int64_t>(128, n / 256);
+    if (std::max(cells, least) < target) {
+      target = std::max(cells, least);
+      fine = true;
+    }
+  }
   const int nc = C > 0 ? C : 1;
   int64_t start = 0;
   for (int k = 0; k < nc; ++k) {
     const int64_t end = C > 0 ? (int64_t)ends[k] : n;
     const int64_t len = end - start;
     const int64_t pieces = (len + target - 1) / target;
+    // short ranges meet on block boundaries: a block that two ranges share is
+    // computed twice
+    auto cut = [&](int64_t q) {
+      const int64_t c = start + len * q / pieces;
+      return fine && q > 0 && q < pieces ? std::max(start, c & ~int64_t(15)) : c;
+    };
     for (int64_t q = 0; q < pieces; ++q) {
-      ch.c0.push_back(start + len * q / pieces);
-      ch.c1.push_back(start + len * (q + 1) / pieces);
+      ch.c0.push_back(cut(q));
+      ch.c1.push_back(cut(q + 1));
       ch.cl.push_back(k);
     }
     start = end;
@@ -1911,7 +1936,8 @@ int run_setup(devil_ctx* ctx, const devil_problem* pr, devil_outputs* out, ProbR
     }
   }
   ctx->aligned_copy = r.dev_counts != pr->counts;
-  if ((rc = build_chunks(ctx, n, C > 0 ? r.ends_h.data() : nullptr, C, r.chunks))) return rc;
+  if ((rc = build_chunks(ctx, n, C > 0 ? r.ends_h.data() : nullptr, C,
+                         r.mixed && C > 0 ? 0 : r.batch, r.chunks))) return rc;
   DV_ALLOC(r.post, sizeof(double) * post_part_doubles(r.tl.td, r.chunks, r.batch));
   r.eps = (double)(float)pr->tolerance;  // src/beta.cpp:25 float eps
   if ((rc = build_init_tile(ctx, r.d, r.dd, r.tl.td, pr->disp_init ? 0 : 1, r.init_mode, r.ih)))
@@ -2886,7 +2912,7 @@ int devil_estimate_dispersion(devil_ctx* ctx, const void* counts, int32_t dtype,
   InitHost ih;
   if ((rc = build_init_tile(ctx, d, dd, td, 1, dv::kInitNone, ih))) return rc;
   ChunkHost chunks;
-  if ((rc = build_chunks(ctx, n, nullptr, 0, chunks))) return rc;
+  if ((rc = build_chunks(ctx, n, nullptr, 0, G, chunks))) return rc;
   DevBuf part;
   DV_ALLOC(part, sizeof(double) * (size_t)((G + 15) / 16) * chunks.ct.nchunk * 16 * 20);
   dv::Counts c{counts, dtype, ld};
@@ -2916,7 +2942,7 @@ int devil_init_beta(devil_ctx* ctx, const void* counts, int32_t dtype, int64_t G
   InitHost ih;
   if ((rc = build_init_tile(ctx, d, dd, td, 0, init_mode, ih))) return rc;
   ChunkHost chunks;
-  if ((rc = build_chunks(ctx, n, nullptr, 0, chunks))) return rc;
+  if ((rc = build_chunks(ctx, n, nullptr, 0, G, chunks))) return rc;
   DevBuf tmp, part;
   DV_ALLOC(tmp, sizeof(double) * G * p);
   DV_ALLOC(part, sizeof(double) * (size_t)((G + 15) / 16) * chunks.ct.nchunk * 16 * 20);
@@ -2981,7 +3007,7 @@ int devil_mom_dispersion(devil_ctx* ctx, const void* counts, int32_t dtype, int6
   TileHost th;
   if ((rc = tile_from_device(ctx, X, offset, n, p, th))) return rc;
   ChunkHost chunks;
-  if ((rc = build_chunks(ctx, n, nullptr, 0, chunks))) return rc;
+  if ((rc = build_chunks(ctx, n, nullptr, 0, G, chunks))) return rc;
   DevBuf bg, post;
   DV_ALLOC(bg, sizeof(double) * G * p);
   DV_ALLOC(post, sizeof(double) * post_part_doubles(th.td, chunks, G));
@@ -3047,7 +3073,7 @@ int devil_bread_meat(devil_ctx* ctx, const void* counts, int32_t dtype, int64_t 
   TileHost th;
   if ((rc = tile_from_device(ctx, X, offset, n, p, th))) return rc;
   ChunkHost chunks;
-  if ((rc = build_chunks(ctx, n, ends_h.data(), n_clusters, chunks))) return rc;
+  if ((rc = build_chunks(ctx, n, ends_h.data(), n_clusters, G, chunks))) return rc;
   DevBuf bg, post;
   DV_ALLOC(bg, sizeof(double) * G * p);
   DV_ALLOC(post, sizeof(double) * post_part_doubles(th.td, chunks, G));
@@ -3075,7 +3101,7 @@ int devil_sandwich_hc0(devil_ctx* ctx, const void* counts, int32_t dtype, int64_
   TileHost th;
   if ((rc = tile_from_device(ctx, X, offset, n, p, th))) return rc;
   ChunkHost chunks;
-  if ((rc = build_chunks(ctx, n, nullptr, 0, chunks))) return rc;
+  if ((rc = build_chunks(ctx, n, nullptr, 0, G, chunks))) return rc;
   DevBuf bg, post;
   DV_ALLOC(bg, sizeof(double) * G * p);
   DV_ALLOC(post, sizeof(double) * post_part_doubles(th.td, chunks, G, true));

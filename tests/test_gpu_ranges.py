@@ -1,0 +1,68 @@
+"""The init and post-IRLS passes on the short cell ranges of fits with few
+genes, and the t tail of test_de, against the oracle.
+
+Bars: those of the FP64 path (test_gpu_parity.py), theta / bread / sandwich
+within 1e-8 relative.  The t tail's continued fraction loses up to about
+df * 2^-53 (its partial sums cancel to 1 / df of their terms), on both sides:
+log p within 1e-12 + 4e-16 df."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+
+
+@pytest.fixture(scope="module")
+def dv():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    import devil_amd
+    devil_amd.lib()
+    return devil_amd
+
+
+def close(a, b, what):
+    a, b = np.asarray(a.cpu()), np.asarray(b)
+    scale = np.abs(b).reshape(len(b), -1).max(1).reshape((-1,) + (1,) * (b.ndim - 1))
+    err = np.abs(a - b) / np.maximum(scale, 1e-12)
+    assert np.all(np.isfinite(err)) and err.max() <= 1e-8, f"{what}: {err.max():.2e}"
+
+
+@pytest.mark.parametrize("G,sizes", [
+    (16, None), (17, None), (1, None), (300, None),
+    (16, [1, 15, 16, 17, 127, 128, 129, 2067]),  # patients shorter than a block and a range
+    (40, [5, 2400, 95])])
+def test_short_ranges(dv, orc, G, sizes):
+    r = np.random.default_rng(G)
+    n = 2500 if sizes is None else sum(sizes)
+    X = np.column_stack([np.ones(n), r.uniform(size=n) < 0.5, r.normal(size=n)])
+    B = np.column_stack([r.normal(1, 0.5, G), r.normal(0, 0.5, G), r.normal(0, 0.1, G)])
+    sf = np.exp(r.normal(0, 0.3, n))
+    mu = sf * np.exp(B @ X.T)
+    Y = r.poisson(r.gamma(2.0, mu / 2.0)).astype(np.int32)
+    lab = None if sizes is None else np.repeat(np.arange(len(sizes)), sizes)
+    ends = None if sizes is None else np.cumsum(sizes).astype(np.int32)
+    print(f"[case] G={G} n={n} patients={sizes}", flush=True)
+    fit = dv.fit_devil(torch.as_tensor(Y, device="cuda"), X, size_factors=sf, clusters=lab)
+    ref = orc.cpu_fit(Y.astype(np.float64), X, np.log(sf), od_mode=orc.OD_MOM,
+                      clusters_ends=ends)
+    np.testing.assert_array_equal(fit["iterations"]["beta_iters"].cpu(), ref["beta_iters"])
+    close(fit["beta"], ref["beta"], "beta")
+    close(fit["overdispersion"], ref["theta"], "theta")
+    close(fit["beta_sandwiches_null"], ref["bread"], "bread")
+    if sizes is not None:
+        close(fit["beta_sandwiches"], ref["sandwich"], "sandwich")
+
+
+@pytest.mark.parametrize("n", [3, 20, 500, 5000, 100000])
+def test_t_tail(dv, orc, n):
+    t = np.concatenate([np.exp(np.linspace(-12, 6, 600)), [0.0, 1.0, 1.8, 2.0]])
+    G = len(t)
+    one = np.ones((G, 1, 1))
+    fit = dict(beta=t[:, None], beta_sandwiches_null=one, design_matrix=np.ones((n, 1)))
+    lp = dv.test_de(fit, [1.0])["log_pval"]
+    ref = orc.de_test(t[:, None], one, None, n, [1.0])["log_pval"]
+    err = np.abs(lp - ref) / np.maximum(1.0, np.abs(ref))
+    print(f"[case] t tail df={n - 2} worst {err.max():.2e}", flush=True)
+    assert np.all(np.isfinite(err)) and err.max() <= 1e-12 + 4e-16 * n
