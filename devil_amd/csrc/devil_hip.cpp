@@ -678,9 +678,18 @@ struct TileHost {
   dv::TileDesign tdm{};  // mixed design (td for FP32, 32-cell steps for bf16)
   const double* X = nullptr;    // device n x p design, column-major
   const double* off = nullptr;  // device offsets
+  int intercept = 0;            // column 0 of X is all ones
   int mixed = kMixedNone;
   DevBuf spec, specm, Xp, offp, eop, Kp, Xf, offf, Kf, xab, offl, kg, kh, kh2;
 };
+
+// The FP64 IRLS takes one workgroup per gene where the design stays in an
+// XCD's L2 (4 MB, shared with the counts of 32 CUs' genes).
+constexpr int64_t kGeneDesignBytes = (int64_t)2 << 20;
+
+bool gene_path(const TileHost& tl, int p) {
+  return (int64_t)sizeof(double) * (p + 1) * tl.td.n <= kGeneDesignBytes;
+}
 
 // Xd, offd, eod: device n x p X, offset and exp(offset).
 int make_tile(devil_ctx* ctx, const double* Xd, const double* offd, const double* eod,
@@ -715,6 +724,11 @@ int make_tile(devil_ctx* ctx, const double* Xd, const double* offd, const double
   td.offp = th.offp.as<double>();
   td.eop = th.eop.as<double>();
   td.Kp = th.Kp.as<double>();
+  // x_0 x_0 == x_0 makes x_0 one or zero; summing to n, it is one everywhere
+  const int c0 = td.kidx_lin[0];
+  th.intercept = c0 >= 0 && td.ksum[c0] == (double)n && td.kidx_pair[0] == c0;
+  for (int b = 0; b < p; ++b)
+    if (td.kidx_pair[b] != td.kidx_lin[b]) th.intercept = 0;
   if (f32) {
     th.tdm = td;
     th.tdm.Xf = th.Xf.as<float>();
@@ -983,6 +997,35 @@ dv::TileDesign round_shape(const dv::TileDesign& td, int nA, int tiles_per_wg,
   return (tr.nchunk > td.nchunk && tr.nchunk <= cap) ? tr : td;
 }
 
+// An FP64 round of at most kCellsGenes genes runs one gene and chunk per
+// wavefront (launch_irls_cells): enough chunks for kCellsRoundWaves wavefronts
+// (eight a SIMD), of at least kMinCells cells each.  The line: 300 genes x
+// 200001 cells, p = 5, spend 2.66 / 2.17 / 1.91 / 2.10 / 2.26 ms in the
+// accumulates with it at 16 / 48 / 128 / 256 / 512 genes, 4000 x 500000,
+// p = 8, 65.3 / 65.7 / 66.1 / 66.0 / 68.5 ms.
+constexpr int64_t kCellsRoundWaves = 8192;
+constexpr int64_t kMinCells = 256;
+constexpr int kCellsGenes = 96;
+
+dv::TileDesign fp64_shape(const dv::TileDesign& td, int64_t nA, size_t part_cap) {
+  if (nA <= 0 || nA > kCellsGenes) return round_shape(td, (int)nA, 4, part_cap);
+  const int64_t cap = (int64_t)(part_cap / ((size_t)((nA + 15) / 16) * 16 * td.ncp));
+  int64_t want = std::min({(kCellsRoundWaves + nA - 1) / nA, kMaxRoundChunks, cap});
+  if (want >= 8) want -= want % 8;  // set_chunks rounds the count up to a multiple of 8
+  dv::TileDesign tr = td;
+  set_chunks(tr, std::max(kMinCells / 16, (td.nblk + want - 1) / want));
+  return tr;  // tr.nchunk <= want <= cap
+}
+
+hipError_t launch_fp64_accum(hipStream_t s, const TileHost& tl, const dv::TileDesign& td,
+                             dv::Counts c, int p, const int32_t* list, const int32_t* nlist,
+                             int bound, const double* beta, const double* kvec, double* part) {
+  if (bound > kCellsGenes)
+    return dv::launch_irls_accum(s, td, c, p, list, nlist, bound, beta, kvec, part);
+  return dv::launch_irls_cells(s, td, c, p, tl.intercept, tl.X, tl.off, list, nlist, bound, beta,
+                               kvec, part);
+}
+
 // Pinned host slots and events through which irls_rounds reads the active
 // counts (made on a context's first fit).
 int round_sync_setup(devil_ctx* ctx) {
@@ -1030,11 +1073,15 @@ int irls_rounds(devil_ctx* ctx, const TileHost& tl, bool mixed, dv::Counts c, in
   volatile int32_t* slot = ctx->round_counts;
   DevBuf red;
   DV_ALLOC(red, sizeof(double) * kSplitTiles * kSplitSlices * 16 * tfull.ncp);
+  auto shape = [&](int genes) {
+    return mixed ? round_shape(tfull, genes, tiles_per_wg, part_cap)
+                 : fp64_shape(tfull, genes, part_cap);
+  };
   // one round over list (a, na) into (b, nb), its next count copied to *out
   auto queue_round = [&](const dv::TileDesign& td, int bound, int32_t* a, int32_t* na,
                          int32_t* b, int32_t* nb, int32_t* out) -> int {
     if (!mixed)
-      DV_HIP(dv::launch_irls_accum(s, td, c, p, a, na, bound, beta, kvec, part));
+      DV_HIP(launch_fp64_accum(s, tl, td, c, p, a, na, bound, beta, kvec, part));
     else
       DV_HIP(launch_mixed_accum(tl.mixed, s, td, c, p, a, na, bound, beta, kvec, part));
     DV_HIP(dv::launch_fill_i32(s, nb, 1, 0));
@@ -1084,7 +1131,7 @@ int irls_rounds(devil_ctx* ctx, const TileHost& tl, bool mixed, dv::Counts c, in
       count.push_back((int)slot[(k - 1) & 1]);  // round k's list
       const int gb = count[k];
       if (gb <= 0) break;
-      const dv::TileDesign td = round_shape(tfull, gb, tiles_per_wg, part_cap);
+      const dv::TileDesign td = shape(gb);
       hipGraph_t g[2] = {nullptr, nullptr};
       hipGraphExec_t ge[2] = {nullptr, nullptr};
       auto cleanup = [&]() {
@@ -1143,12 +1190,12 @@ int irls_rounds(devil_ctx* ctx, const TileHost& tl, bool mixed, dv::Counts c, in
       graphed = true;
       break;
     }
-    const dv::TileDesign td = round_shape(tfull, bound, tiles_per_wg, part_cap);
+    const dv::TileDesign td = shape(bound);
     const size_t nrec = ctx->launches.size();
     {
       LaunchTimer lt(ctx, kind, 0.0);
       if (!mixed)
-        DV_HIP(dv::launch_irls_accum(s, td, c, p, cur, ncur, bound, beta, kvec, part));
+        DV_HIP(launch_fp64_accum(s, tl, td, c, p, cur, ncur, bound, beta, kvec, part));
       else
         DV_HIP(launch_mixed_accum(tl.mixed, s, td, c, p, cur, ncur, bound, beta, kvec, part));
     }
@@ -1251,28 +1298,15 @@ int driver_rounds(devil_ctx* ctx, const dv::TileDesign& tfull, size_t part_cap, 
   return DEVIL_OK;
 }
 
-// The FP64 IRLS takes one workgroup per gene where the design stays in an
-// XCD's L2 (4 MB, shared with the counts of 32 CUs' genes).
-constexpr int64_t kGeneDesignBytes = (int64_t)2 << 20;
-
-bool gene_path(const TileHost& tl, int p) {
-  return (int64_t)sizeof(double) * (p + 1) * tl.td.n <= kGeneDesignBytes;
-}
-
-dv::GeneDesign gene_design(const TileHost& tl, int p) {
+dv::GeneDesign gene_design(const TileHost& tl) {
   dv::GeneDesign gd{};
   gd.n = tl.td.n;
   gd.X = tl.X;
   gd.off = tl.off;
+  gd.intercept = tl.intercept;
   std::memcpy(gd.kidx_pair, tl.td.kidx_pair, sizeof(gd.kidx_pair));
   std::memcpy(gd.kidx_lin, tl.td.kidx_lin, sizeof(gd.kidx_lin));
   std::memcpy(gd.ksum, tl.td.ksum, sizeof(gd.ksum));
-  // x_0 x_b == x_b for every b makes x_0 one or zero where it matters; summing
-  // to n, it is one everywhere
-  const int c0 = tl.td.kidx_lin[0];
-  gd.intercept = c0 >= 0 && tl.td.ksum[c0] == (double)tl.td.n;
-  for (int b = 0; b < p; ++b)
-    if (tl.td.kidx_pair[b] != tl.td.kidx_lin[b]) gd.intercept = 0;
   return gd;
 }
 
@@ -1287,7 +1321,7 @@ int run_irls_gene(devil_ctx* ctx, const TileHost& tl, dv::Counts c, int p, const
   DV_ALLOC(next, sizeof(int32_t));
   {
     LaunchTimer lt(ctx, DEVIL_KERNEL_IRLS_FP64, 0.0);
-    DV_HIP(dv::launch_irls_gene(s, gene_design(tl, p), c, p, list, ngenes, next.as<int32_t>(),
+    DV_HIP(dv::launch_irls_gene(s, gene_design(tl), c, p, list, ngenes, next.as<int32_t>(),
                                 beta, kvec, max_iter, eps, iters, status));
   }
   if (ctx->launches.size() > nrec) {  // timing: the bytes follow from the iterations
@@ -1331,7 +1365,11 @@ int run_irls_tiled(devil_ctx* ctx, const TileHost& tl, dv::Counts c, int64_t G, 
   size_t part_per_tile = (size_t)td.nchunk * 16 * td.ncp;
   if (mixed) part_per_tile = std::max(part_per_tile, (size_t)tdm.nchunk * 16 * tdm.ncp);
   const size_t part_cap = (size_t)ntile * part_per_tile;
-  DV_ALLOC(part, sizeof(double) * part_cap);
+  // the FP64 rounds of few genes may need more (the mixed rounds' chunks, over
+  // which the pair columns are summed in FP32, follow part_cap)
+  const size_t cap64 = std::max<size_t>(
+      part_cap, (size_t)((kCellsGenes + 15) / 16) * 16 * td.ncp * kMaxRoundChunks);
+  DV_ALLOC(part, sizeof(double) * cap64);
   int32_t* c0 = cnt.as<int32_t>();
   DV_HIP(dv::launch_iota(s, act0.as<int32_t>(), (int)G));
   DV_HIP(dv::launch_fill_i32(s, c0, 1, (int32_t)G));
@@ -1339,7 +1377,7 @@ int run_irls_tiled(devil_ctx* ctx, const TileHost& tl, dv::Counts c, int64_t G, 
   if (!mixed)
     return irls_rounds(ctx, tl, false, c, p, beta, kvec, max_iter, eps, iters, status,
                        act0.as<int32_t>(), act1.as<int32_t>(), c0, c0 + 1, (int)G,
-                       part.as<double>(), part_cap, nullptr, nullptr);
+                       part.as<double>(), cap64, nullptr, nullptr);
   DevBuf bprev;
   DV_ALLOC(rep, sizeof(int32_t) * G);
   DV_ALLOC(beta0, sizeof(double) * G * p);
@@ -1367,7 +1405,7 @@ int run_irls_tiled(devil_ctx* ctx, const TileHost& tl, dv::Counts c, int64_t G, 
     else
       rc = irls_rounds(ctx, tl, false, c, p, beta, kvec, max_iter, eps, iters, status,
                        rep.as<int32_t>(), act1.as<int32_t>(), nrep, c0 + 3, nr,
-                       part.as<double>(), part_cap, nullptr, nullptr);
+                       part.as<double>(), cap64, nullptr, nullptr);
     if (rc) return rc;
   }
   // The mixed trajectory leaves ~5e-7 absolute on beta; where a coefficient
@@ -1383,9 +1421,9 @@ int run_irls_tiled(devil_ctx* ctx, const TileHost& tl, dv::Counts c, int64_t G, 
   DV_HIP(hipStreamSynchronize(s));
   ctx->polished += np;
   if (np == 0) return DEVIL_OK;
-  const dv::TileDesign td1 = round_shape(td, np, 4, part_cap);
-  DV_HIP(dv::launch_irls_accum(s, td1, c, p, list, c0, np, bprev.as<double>(), kvec,
-                               part.as<double>()));
+  const dv::TileDesign td1 = fp64_shape(td, np, cap64);
+  DV_HIP(launch_fp64_accum(s, tl, td1, c, p, list, c0, np, bprev.as<double>(), kvec,
+                           part.as<double>()));
   DV_HIP(dv::launch_irls_update(s, td1, p, list, c0, np, part.as<double>(), beta, kvec, max_iter,
                                 eps, iters, status, act1.as<int32_t>(), c0 + 1, 0.0, nullptr,
                                 nullptr, bprev.as<double>(), 1));

@@ -214,6 +214,14 @@ hipError_t launch_irls_gene(hipStream_t s, const GeneDesign& gd, Counts c, int p
                             const double* kvec, int max_iter, double eps, int32_t* iters,
                             int32_t* status);
 
+// FP64 IRLS accumulate of a round of few genes, one gene and chunk per
+// wavefront (kernels_cells.hip); X, off: the caller's layout, td: the chunks
+// and columns.  part is laid out as launch_irls_accum's.
+hipError_t launch_irls_cells(hipStream_t s, const TileDesign& td, Counts c, int p, int intercept,
+                             const double* X, const double* off, const int32_t* active,
+                             const int32_t* nactive, int nA_bound, const double* beta,
+                             const double* kvec, double* part);
+
 // One problem's share of a joint round (kernels_tile.hip): its round shape,
 // counts, active list and outputs, its workgroups of the accumulate grid and
 // its blocks of the update grid.

@@ -29,52 +29,10 @@
 #include "../../include/devil_hip.h"
 #include "device_common.hpp"
 #include "kernels.hpp"
+#include "lane_sums.hpp"
 #include "tile_common.hpp"
 
 namespace dv {
-
-// Lane sums of V values: after reduce_scatter the lane with index parts
-// scatter_index holds the wave's sum of value scatter_index + i in v[i],
-// i < scatter_left(V).  Each step halves the values a lane holds and pairs
-// lanes 32, 16, 8, 4, 2, 1 apart, so the 64-lane sums of V values take about
-// V exchanges instead of 6 V.
-__host__ __device__ constexpr int scatter_left(int V) {
-  for (int i = 0; i < 6; ++i) V = (V + 1) / 2;
-  return V;
-}
-
-template <int M, int MASK>
-__device__ __forceinline__ void scatter_step(double* v, int lane) {
-  constexpr int H = (M + 1) / 2;
-  const bool up = lane & MASK;
-#pragma unroll
-  for (int i = 0; i < H; ++i) {
-    const double lo = v[i], hi = H + i < M ? v[H + i] : 0.0;
-    const double keep = up ? hi : lo, send = up ? lo : hi;
-    v[i] = keep + __shfl_xor(send, MASK, 64);
-  }
-  if constexpr (MASK > 1) scatter_step<H, MASK / 2>(v, lane);
-}
-
-// first value index of this lane's sums; *valid[i] false where the lane's
-// i-th entry stands for no value
-template <int V>
-__device__ __forceinline__ int scatter_index(int lane, int i) {
-  int m[6], v = V;
-  for (int k = 0; k < 6; ++k) {
-    m[k] = v;
-    v = (v + 1) / 2;
-  }
-  int pos = i;
-  for (int k = 5; k >= 0; --k) {
-    const int half = (m[k] + 1) / 2;
-    if (lane & (32 >> k)) {
-      pos += half;
-      if (pos >= m[k]) return -1;
-    }
-  }
-  return pos;
-}
 
 template <int P, int NG, typename CT>
 struct GeneOps {

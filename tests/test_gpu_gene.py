@@ -80,3 +80,12 @@ def test_iteration_limit(dv, orc):
 
 def test_more_genes_than_workgroups(dv, orc):
     check(dv, orc, *problem(5000, 300, 2))
+
+
+@pytest.mark.parametrize("p,intercept", [(2, True), (3, False), (6, True), (8, False), (10, True)])
+@pytest.mark.parametrize("G", [1, 5, 96, 97, 200])
+def test_round_kernels(dv, orc, G, p, intercept):
+    """Rows too long for the gene kernel: one gene per wavefront up to 96
+    active genes, 16-gene tiles above."""
+    Y, X, sf = problem(G, (2 << 20) // (8 * (p + 1)) + 77, p, intercept)
+    check(dv, orc, Y, X, sf)
