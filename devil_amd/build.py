@@ -22,7 +22,7 @@ ROOT = os.path.dirname(HERE)
 
 SOURCES = ["kernels_epilogue.hip", "kernels_tile.hip", "kernels_mle.hip", "kernels_post.hip",
            "kernels_design.hip", "kernels_prep.hip", "kernels_newod.hip", "kernels_gene.hip",
-           "kernels_cells.hip",
+           "kernels_cells.hip", "kernels_irls64.hip",
            "devil_hip.cpp"]
 
 COMMON = [

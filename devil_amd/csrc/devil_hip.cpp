@@ -664,6 +664,7 @@ void shape_design(const ColPlan& cp, int64_t n, int p, int cells_per_block, dv::
   const int ncol = std::max<int>(1, (int)cp.spec.size());
   td.nt = (ncol + 15) / 16;
   td.ncp = 16 * td.nt;
+  td.ncol = ncol;
   td.n = n;
   td.nblk = (n + cells_per_block - 1) / cells_per_block;
   const int64_t min_blocks = std::max<int64_t>(1, chunk_cells / cells_per_block);

@@ -33,6 +33,7 @@ struct TileDesign {
   int nchunk;            // chunks; partial sums are kept per chunk
   int nt;                // 16-column tiles of K
   int ncp;               // 16 * nt
+  int ncol;              // columns of K in use
   const double* Xp;      // [blk][j][lane] = X[16 blk + pi(lane%16)][4 j + lane/16] (0-padded),
                          // pi(m) = 4 (m % 4) + m / 4
   const double* offp;    // off padded with zeros to 16 nblk

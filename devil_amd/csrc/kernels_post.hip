@@ -92,9 +92,10 @@ __device__ __forceinline__ void mom_tile_chunk(const TileDesign& td, ChunkTable 
   }
 }
 
-// HC: also the HC0 meat sum, sum_i r_i^2 x_i x_i' with r = (y - mu) / (1 + theta mu)
+// SC 0: bread only; 1: also the score sums sum_i r_i x_i (clustered meat);
+// 2: also the HC0 meat sum, sum_i r_i^2 x_i x_i' with r = (y - mu) / (1 + theta mu)
 // (src/variance.cpp:64-85, 157-178), in ncp more partial columns.
-template <int P, typename CT, bool VEC, bool HC>
+template <int P, int SC, int VC, typename CT, bool VEC>
 __device__ __forceinline__ void bread_tile_chunk(const TileDesign& td, ChunkTable ct,
                                                  const CT* __restrict__ Y, int64_t ld,
                                                  int64_t G, const double* __restrict__ beta,
@@ -102,13 +103,15 @@ __device__ __forceinline__ void bread_tile_chunk(const TileDesign& td, ChunkTabl
                                                  int chunk, double* __restrict__ part,
                                                  const double* __restrict__ e2) {
   constexpr int NJ = (P + 3) / 4;
-  constexpr int NTMAX = ((P * (P + 1)) / 2 + P + 15) / 16;
+  constexpr bool HC = SC == 2;
+  constexpr int NTMAX = mfma_tiles<P, VC>();
+  constexpr int NTA = NTMAX > 0 ? NTMAX : 1;
   const int lane = threadIdx.x & 63;
   const int s = lane & 15, h = lane >> 4;
   const int64_t g0 = (int64_t)tile * 16 + s;
   const bool live = g0 < G;
   const int64_t g = live ? g0 : (int64_t)tile * 16;
-  const int NT = td.nt;
+  const int NT = VC > 0 ? td.ncol / 16 : td.nt;
   double bpos[NJ];
 #pragma unroll
   for (int j = 0; j < NJ; ++j) {
@@ -118,16 +121,19 @@ __device__ __forceinline__ void bread_tile_chunk(const TileDesign& td, ChunkTabl
   const double th = live ? theta[g] : 0.0;
   const CT* yrow = Y + g * ld;
   const CT* yh = yrow + 4 * h;
-  d4 aw[NTMAX], ah[HC ? NTMAX : 1], ar;
+  d4 aw[NTA], ah[HC ? NTA : 1], ar;
+  double avw[VC > 0 ? VC : 1], avh[VC > 0 ? VC : 1], avr[VC > 0 ? VC : 1];
+#pragma unroll
+  for (int v = 0; v < VC; ++v) avw[v] = avh[v] = avr[v] = 0.0;
 #pragma unroll
   for (int t = 0; t < NTMAX; ++t) aw[t] = d4{0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-  for (int t = 0; t < (HC ? NTMAX : 1); ++t) ah[t] = d4{0.0, 0.0, 0.0, 0.0};
+  for (int t = 0; t < (HC ? NTA : 1); ++t) ah[t] = d4{0.0, 0.0, 0.0, 0.0};
   ar = d4{0.0, 0.0, 0.0, 0.0};
   const int64_t c0 = ct.c0[chunk], c1 = ct.c1[chunk];
   const int64_t b0 = c0 / 16, b1 = c0 < c1 ? (c1 + 15) / 16 : b0;
   typedef TileBlock<NJ, NTMAX, CT> Blk;  // off holds exp(offset)
-  auto body = [&](const Blk& cur, int64_t b) {
+  auto body = [&](const Blk& cur, const VCols<VC>& kv, int64_t b) {
     d4 eta = d4{0.0, 0.0, 0.0, 0.0};
 #pragma unroll
     for (int j = 0; j < NJ; ++j) eta = mfma16x16x4(cur.xa[j], bpos[j], eta);
@@ -150,25 +156,38 @@ __device__ __forceinline__ void bread_tile_chunk(const TileDesign& td, ChunkTabl
         for (int r = 0; r < 4; ++r) aw[t] = mfma16x16x4(w[r], cur.kb[t][r], aw[t]);
       }
     }
+    add_vcols<VC>(w, kv.k, avw);
     if constexpr (HC) {
+      double r2[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) r2[r] = rr[r] * rr[r];
 #pragma unroll
       for (int t = 0; t < NTMAX; ++t) {
         if (t < NT) {
 #pragma unroll
-          for (int r = 0; r < 4; ++r) ah[t] = mfma16x16x4(rr[r] * rr[r], cur.kb[t][r], ah[t]);
+          for (int r = 0; r < 4; ++r) ah[t] = mfma16x16x4(r2[r], cur.kb[t][r], ah[t]);
         }
       }
+      add_vcols<VC>(r2, kv.k, avh);
     }
+    // the design columns are among the first 16 columns
+    if constexpr (SC == 1) {
+      if (NTMAX > 0 && NT > 0) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) ar = mfma16x16x4(rr[r], cur.kb[0][r], ar);
+        for (int r = 0; r < 4; ++r) ar = mfma16x16x4(rr[r], cur.kb[0][r], ar);
+      } else {
+        add_vcols<VC>(rr, kv.k, avr);
+      }
+    }
   };
+  auto load_own = [&](int64_t b, VCols<VC>& o) { load_vcols<VC>(td, b, h, NT, o.k); };
   auto load = [&](int64_t b, Blk& o) {
     load_tile_block<NJ, NTMAX, CT, VEC>(td, yh, b, lane, h, NT, td.eop, o);
   };
   auto load_tail = [&](int64_t b, Blk& o) {
     load_tile_block_tail<NJ, NTMAX, CT>(td, yrow, b, lane, h, NT, td.eop, o);
   };
-  pipeline<Blk>(b0, min(b1, td.n / 16), b1, load, load_tail, body);
+  pipeline_own<Blk, VCols<VC>>(b0, min(b1, td.n / 16), b1, load, load_tail, load_own, body);
   // register r holds gene slot h + 4 r, column 16 t + s
   const int W = td.ncp + 16 + (HC ? td.ncp : 0);
   double* out = part + ((int64_t)tile * ct.nchunk + chunk) * 16 * W;
@@ -179,8 +198,15 @@ __device__ __forceinline__ void bread_tile_chunk(const TileDesign& td, ChunkTabl
       for (int r = 0; r < 4; ++r) out[(h + 4 * r) * W + 16 * t + s] = aw[t][r];
     }
   }
+  store_vcols<VC>(td, h, NT, avw, out + s * W + 16 * NT);
+  if constexpr (SC == 1) {
+    if (NTMAX > 0 && NT > 0) {
 #pragma unroll
-  for (int r = 0; r < 4; ++r) out[(h + 4 * r) * W + td.ncp + s] = ar[r];
+      for (int r = 0; r < 4; ++r) out[(h + 4 * r) * W + td.ncp + s] = ar[r];
+    } else {
+      store_vcols<VC>(td, h, NT, avr, out + s * W + td.ncp);
+    }
+  }
   if constexpr (HC) {
 #pragma unroll
     for (int t = 0; t < NTMAX; ++t) {
@@ -189,6 +215,7 @@ __device__ __forceinline__ void bread_tile_chunk(const TileDesign& td, ChunkTabl
         for (int r = 0; r < 4; ++r) out[(h + 4 * r) * W + td.ncp + 16 + 16 * t + s] = ah[t][r];
       }
     }
+    store_vcols<VC>(td, h, NT, avh, out + s * W + td.ncp + 16 + 16 * NT);
   }
 }
 
@@ -235,7 +262,7 @@ __global__ __launch_bounds__(256) void k_mom_finish(ChunkTable ct, int64_t G, in
   if (status && !(den > 0.0)) status[g] |= DEVIL_GENE_MOM_DEN0;
 }
 
-template <int P, bool HC>
+template <int P, int SC, int VC>
 __global__ __launch_bounds__(256) void k_bread_accum(TileDesign td, ChunkTable ct, Counts c,
                                                      int64_t G, const double* __restrict__ beta,
                                                      const double* __restrict__ theta,
@@ -250,8 +277,8 @@ __global__ __launch_bounds__(256) void k_bread_accum(TileDesign td, ChunkTable c
   if ((int64_t)tile * 16 >= G) return;
   with_counts(c, [&](auto Y, auto vec) {
     typedef std::remove_cv_t<std::remove_pointer_t<decltype(Y)>> CT;
-    bread_tile_chunk<P, CT, decltype(vec)::value, HC>(td, ct, Y, c.ld, G, beta, theta, tile,
-                                                      chunk, part, e2);
+    bread_tile_chunk<P, SC, VC, CT, decltype(vec)::value>(td, ct, Y, c.ld, G, beta, theta, tile,
+                                                          chunk, part, e2);
   });
 }
 
@@ -606,26 +633,47 @@ __global__ __launch_bounds__(256) void k_init_finish(InitTile it, ChunkTable ct,
     default: return hipErrorInvalidValue;                                           \
   }
 
-// the same dispatch for kernels with a second (bool) template argument
-#define DV_POST_P2_CASE(P_, KERNEL, B, GRID, BLOCK, STREAM, ...)    \
-  case P_: {                                                        \
-    auto k_ = KERNEL<P_, B>;                                        \
-    hipLaunchKernelGGL(k_, GRID, BLOCK, 0, STREAM, __VA_ARGS__);    \
-  } break;
-#define DV_POST_P2(p, KERNEL, B, GRID, BLOCK, STREAM, ...)                     \
-  switch (p) {                                                                \
-    DV_POST_P2_CASE(1, KERNEL, B, GRID, BLOCK, STREAM, __VA_ARGS__)           \
-    DV_POST_P2_CASE(2, KERNEL, B, GRID, BLOCK, STREAM, __VA_ARGS__)           \
-    DV_POST_P2_CASE(3, KERNEL, B, GRID, BLOCK, STREAM, __VA_ARGS__)           \
-    DV_POST_P2_CASE(4, KERNEL, B, GRID, BLOCK, STREAM, __VA_ARGS__)           \
-    DV_POST_P2_CASE(5, KERNEL, B, GRID, BLOCK, STREAM, __VA_ARGS__)           \
-    DV_POST_P2_CASE(6, KERNEL, B, GRID, BLOCK, STREAM, __VA_ARGS__)           \
-    DV_POST_P2_CASE(7, KERNEL, B, GRID, BLOCK, STREAM, __VA_ARGS__)           \
-    DV_POST_P2_CASE(8, KERNEL, B, GRID, BLOCK, STREAM, __VA_ARGS__)           \
-    DV_POST_P2_CASE(9, KERNEL, B, GRID, BLOCK, STREAM, __VA_ARGS__)           \
-    DV_POST_P2_CASE(10, KERNEL, B, GRID, BLOCK, STREAM, __VA_ARGS__)          \
-    default: return hipErrorInvalidValue;                                     \
+template <int P, int SC>
+hipError_t launch_bread_accum(hipStream_t s, dim3 grid, const TileDesign& td,
+                              const ChunkTable& ct, Counts c, int64_t G, const double* beta,
+                              const double* theta, double* part) {
+  switch (vcols_of(td.ncol)) {
+    case 0:
+      hipLaunchKernelGGL((k_bread_accum<P, SC, 0>), grid, dim3(256), 0, s, td, ct, c, G, beta,
+                         theta, part);
+      break;
+    case 1:
+      hipLaunchKernelGGL((k_bread_accum<P, SC, 1>), grid, dim3(256), 0, s, td, ct, c, G, beta,
+                         theta, part);
+      break;
+    default:
+      hipLaunchKernelGGL((k_bread_accum<P, SC, 2>), grid, dim3(256), 0, s, td, ct, c, G, beta,
+                         theta, part);
   }
+  return hipGetLastError();
+}
+
+template <int SC>
+hipError_t launch_bread_accum_p(int p, hipStream_t s, dim3 grid, const TileDesign& td,
+                                const ChunkTable& ct, Counts c, int64_t G, const double* beta,
+                                const double* theta, double* part) {
+#define DV_BREAD_P(P_) \
+  case P_: return launch_bread_accum<P_, SC>(s, grid, td, ct, c, G, beta, theta, part);
+  switch (p) {
+    DV_BREAD_P(1)
+    DV_BREAD_P(2)
+    DV_BREAD_P(3)
+    DV_BREAD_P(4)
+    DV_BREAD_P(5)
+    DV_BREAD_P(6)
+    DV_BREAD_P(7)
+    DV_BREAD_P(8)
+    DV_BREAD_P(9)
+    DV_BREAD_P(10)
+    default: return hipErrorInvalidValue;
+  }
+#undef DV_BREAD_P
+}
 
 hipError_t launch_mom_tiled(hipStream_t s, const TileDesign& td, const ChunkTable& ct, Counts c,
                             int64_t G, int64_t n, int p, const double* beta, double* part,
@@ -645,13 +693,12 @@ hipError_t launch_bread_tiled(hipStream_t s, const TileDesign& td, const ChunkTa
                               double* sandwich, int32_t* status) {
   if (G <= 0) return hipSuccess;
   const int64_t groups = ((G + 15) / 16 + 3) / 4;
-  if (C < 0) {
-    DV_POST_P2(p, k_bread_accum, true, dim3((unsigned)(groups * ct.nchunk)), dim3(256), s, td,
-               ct, c, G, beta, theta, part);
-  } else {
-    DV_POST_P2(p, k_bread_accum, false, dim3((unsigned)(groups * ct.nchunk)), dim3(256), s, td,
-               ct, c, G, beta, theta, part);
-  }
+  const dim3 grid((unsigned)(groups * ct.nchunk));
+  const hipError_t e =
+      C < 0 ? launch_bread_accum_p<2>(p, s, grid, td, ct, c, G, beta, theta, part)
+      : C > 0 && sandwich ? launch_bread_accum_p<1>(p, s, grid, td, ct, c, G, beta, theta, part)
+                          : launch_bread_accum_p<0>(p, s, grid, td, ct, c, G, beta, theta, part);
+  if (e != hipSuccess) return e;
   DV_POST_P(p, k_bread_finish, dim3((unsigned)G), dim3(64), s, td, ct, G, n, C, part, bread,
             sandwich, status, 0);
   return hipGetLastError();

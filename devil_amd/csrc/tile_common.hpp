@@ -119,6 +119,42 @@ __device__ __forceinline__ void pipeline(int64_t i0, int64_t i1f, int64_t i1, Lo
   }
 }
 
+// pipeline with operands that a step loads for itself (into one of two buffers
+// in turn) before the next step's loads are issued, for what is used late in
+// the step and would cost too many registers to hold a step ahead.
+template <typename Ops, typename Own, typename Load, typename LoadTail, typename LoadOwn,
+          typename Body>
+__device__ __forceinline__ void pipeline_own(int64_t i0, int64_t i1f, int64_t i1, Load&& load,
+                                             LoadTail&& load_tail, LoadOwn&& load_own,
+                                             Body&& body) {
+  if (i0 < i1f) {
+    Ops A, B;
+    load(i0, A);
+    for (int64_t i = i0; i < i1f; i += 2) {
+      Own K;
+      load_own(i, K);
+      load(min(i + 1, i1f - 1), B);
+      body(A, K, i);
+      if (i + 1 >= i1f) break;
+      load_own(i + 1, K);
+      load(min(i + 2, i1f - 1), A);
+      body(B, K, i + 1);
+    }
+  }
+  for (int64_t i = max(i0, i1f); i < i1; ++i) {
+    Ops T;
+    Own K;
+    load_own(i, K);
+    load_tail(i, T);
+    body(T, K, i);
+  }
+}
+
+template <int VC>
+struct VCols {
+  d4 k[VC > 0 ? VC : 1];
+};
+
 // Operands of one 16-cell block for one lane: counts (as stored), the eta
 // A operands, four offsets (log or exp scale, by the caller's table) and the
 // first NTMAX K tiles (none when NTMAX is 0).
@@ -141,11 +177,72 @@ __device__ __forceinline__ void load_tile_tables(const TileDesign& td, int64_t b
   for (int j = 0; j < NJ; ++j) o.xa[j] = xs[j * 64 + lane];
   o.off = reinterpret_cast<const d4*>(offs + b * 16)[h];
   if constexpr (NTMAX > 0) {
-    const d4* ks = reinterpret_cast<const d4*>(td.Kp) + b * NT * 64;
+    const d4* ks = reinterpret_cast<const d4*>(td.Kp) + b * td.nt * 64;
 #pragma unroll
     for (int t = 0; t < NTMAX; ++t) {
-      const int tt = t < NT ? t : NT - 1;  // unused tiles load tile NT - 1 (no branch)
+      const int tt = t < NT ? t : max(NT - 1, 0);  // unused tiles load a used one (no branch)
       o.kb[t] = ks[tt * 64 + lane];
+    }
+  }
+}
+
+// The f64 matrix instruction runs on the vector FP64 units at their rate (64
+// cycles for 1024 products; the two do not overlap), so the padding of the
+// last 16-column tile is time: 4 instructions of 64 cycles per block.  With at
+// most kMaxVCols columns in it they are summed by vector instructions instead,
+// 4 per column and block (VC of them compiled in).  IRLS of 4000 genes x
+// 500000 cells, p = 8 (33 columns): 65.7 -> 57.9 ms; with four columns (1500 x
+// 310683, p = 6: 20) their operands cost the third wave of a SIMD, 13.2 ->
+// 13.9 ms, so three and four stay on a matrix tile.
+constexpr int kMaxVCols = 2;
+
+__host__ __device__ inline int vcols_of(int ncol) {
+  const int rem = ncol % 16;
+  return rem > kMaxVCols ? 0 : rem;
+}
+
+// Matrix tiles of a P-column design with VC vector columns, at most.
+template <int P, int VC>
+__host__ __device__ constexpr int mfma_tiles() {
+  constexpr int most = (P * (P + 1)) / 2 + P;
+  return VC > 0 ? most / 16 : (most + 15) / 16;
+}
+
+// The lane's cells of the vector columns of block b: columns 16 NT + v of K
+// (past the last one, the last again).
+template <int VC>
+__device__ __forceinline__ void load_vcols(const TileDesign& td, int64_t b, int h, int NT,
+                                           d4 (&kv)[VC > 0 ? VC : 1]) {
+  if constexpr (VC > 0) {
+    const int nv = td.ncol - 16 * NT;
+    const d4* ks = reinterpret_cast<const d4*>(td.Kp) + (b * td.nt + NT) * 64 + h * 16;
+#pragma unroll
+    for (int v = 0; v < VC; ++v) kv[v] = ks[min(v, nv - 1)];
+  }
+}
+
+// acc[v] += q' (column v), the lane's four cells
+template <int VC>
+__device__ __forceinline__ void add_vcols(const double (&q)[4], const d4 (&kv)[VC > 0 ? VC : 1],
+                                          double (&acc)[VC > 0 ? VC : 1]) {
+  if constexpr (VC > 0) {
+#pragma unroll
+    for (int v = 0; v < VC; ++v)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[v] = fma(q[r], kv[v][r], acc[v]);
+  }
+}
+
+// out[v] of gene slot s (lanes s, s + 16, s + 32, s + 48 hold its cells)
+template <int VC>
+__device__ __forceinline__ void store_vcols(const TileDesign& td, int h, int NT,
+                                            double (&acc)[VC > 0 ? VC : 1], double* out) {
+  if constexpr (VC > 0) {
+#pragma unroll
+    for (int v = 0; v < VC; ++v) {
+      acc[v] += __shfl_xor(acc[v], 16, 64);
+      acc[v] += __shfl_xor(acc[v], 32, 64);
+      if (h == 0 && v < td.ncol - 16 * NT) out[v] = acc[v];
     }
   }
 }

@@ -66,3 +66,53 @@ def test_t_tail(dv, orc, n):
     err = np.abs(lp - ref) / np.maximum(1.0, np.abs(ref))
     print(f"[case] t tail df={n - 2} worst {err.max():.2e}", flush=True)
     assert np.all(np.isfinite(err)) and err.max() <= 1e-12 + 4e-16 * n
+
+
+@pytest.mark.parametrize("extra", [0, 1, 2, 3])
+@pytest.mark.parametrize("patients", [0, 3])
+def test_vector_columns(dv, orc, extra, patients):
+    """Designs of 16 + extra distinct columns of products (and of two): a last
+    tile of one or two columns is summed by vector instructions, in the IRLS
+    rounds, the bread, the score sums and the HC0 meat."""
+    r = np.random.default_rng(extra)
+    G, n = 130, 45000
+    # 1, b1..bk 0/1 columns, z: distinct columns 1 + k + k (k - 1) / 2 + 1 + k + 1
+    if extra == 0:
+        X = np.column_stack([np.ones(n), r.uniform(size=n) < 0.5])  # 2 columns
+    elif extra == 1:  # 3 indicators of one factor (products zero), 4 covariates: 1+3+4+12+10
+        lv = r.integers(0, 4, n)
+        X = np.column_stack([np.ones(n), lv == 1] + [r.normal(size=n) for _ in range(4)])[:, :6]
+        X[:, 5] = lv == 2  # 1 2 3 z1..z3: 18 columns
+    elif extra == 2:
+        X = np.column_stack([np.ones(n), r.uniform(size=n) < 0.5] +
+                            [r.normal(size=n) for _ in range(6)])  # 33 columns or more
+        X[:, 2] = (r.uniform(size=n) < 0.3) & (X[:, 1] == 0)
+    else:
+        X = r.normal(size=(n, 5)) + 0.2  # 20 columns, no intercept
+    X = X.astype(np.float64)
+    p = X.shape[1]
+    B = np.column_stack([r.normal(0.7, 0.3, G)] + [r.normal(0, 0.1, G) for _ in range(p - 1)])
+    sf = np.exp(r.normal(0, 0.3, n))
+    mu = sf * np.exp(np.clip(B @ X.T, -4, 4))
+    Y = r.poisson(r.gamma(2.0, mu / 2.0)).astype(np.int32)
+    lab = np.sort(r.integers(0, patients, n)) if patients else None
+    ends = None if lab is None else np.cumsum(np.bincount(lab)).astype(np.int32)
+    print(f"[case] vector columns p={p} extra={extra} patients={patients}", flush=True)
+    Yd = torch.as_tensor(Y, device="cuda")
+    fit = dv.fit_devil(Yd, X, size_factors=sf, clusters=lab)
+    ref = orc.cpu_fit(Y.astype(np.float64), X, np.log(sf), od_mode=orc.OD_MOM,
+                      clusters_ends=ends, n_threads=8)
+    np.testing.assert_array_equal(fit["iterations"]["beta_iters"].cpu(), ref["beta_iters"])
+    close(fit["beta"], ref["beta"], "beta")
+    close(fit["beta_sandwiches_null"], ref["bread"], "bread")
+    if patients:
+        close(fit["beta_sandwiches"], ref["sandwich"], "sandwich")
+    else:
+        b, th = fit["beta"].cpu().numpy(), fit["overdispersion"].cpu().numpy()
+        sw = dv.compute_sandwich(X, Yd, b, th, sf)
+        want = []
+        for g in range(0, G, 13):
+            h = orc.compute_hessian(b[g], th[g], Y[g].astype(float), X, sf)
+            m = orc.meat_hc0(X, Y[g].astype(float), b[g], th[g], sf)
+            want.append(h @ m @ h * n)
+        close(sw[::13], np.array(want), "HC0")
