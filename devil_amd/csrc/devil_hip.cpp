@@ -99,6 +99,9 @@ struct devil_ctx {
   int32_t* round_counts = nullptr;  // pinned host slots
   int32_t* round_counts_dev = nullptr;  // the same slots as the device addresses them
   hipEvent_t round_ev[2] = {nullptr, nullptr};
+  // what the design set-up reads back (kernels write it there), see SetupHost
+  void* setup_host = nullptr;
+  void* setup_dev = nullptr;  // the same memory as the device addresses it
   int64_t joined = 0;                 // problems of the last fit in the joint rounds
   // joint rounds of many problems: pinned counts and round descriptors
   void* joint_host = nullptr;
@@ -126,16 +129,20 @@ struct DevBuf {
   void* p = nullptr;
   size_t size = 0;
   BlockCache* cache = nullptr;
+  bool borrowed = false;  // the caller's memory
   DevBuf() = default;
   DevBuf(const DevBuf&) = delete;
   DevBuf& operator=(const DevBuf&) = delete;
-  DevBuf(DevBuf&& o) noexcept : p(o.p), size(o.size), cache(o.cache) { o.p = nullptr; }
+  DevBuf(DevBuf&& o) noexcept : p(o.p), size(o.size), cache(o.cache), borrowed(o.borrowed) {
+    o.p = nullptr;
+  }
   DevBuf& operator=(DevBuf&& o) noexcept {
     if (this != &o) {
       release();
       p = o.p;
       size = o.size;
       cache = o.cache;
+      borrowed = o.borrowed;
       o.p = nullptr;
     }
     return *this;
@@ -143,9 +150,15 @@ struct DevBuf {
   ~DevBuf() { release(); }
   void release() {
     if (!p) return;
-    if (cache) cache->give(p, size);
+    if (borrowed) borrowed = false;
+    else if (cache) cache->give(p, size);
     else (void)hipFree(p);
     p = nullptr;
+  }
+  void borrow(void* ptr) {
+    release();
+    p = ptr;
+    borrowed = ptr != nullptr;
   }
   hipError_t alloc(BlockCache* c, size_t bytes) {
     release();
@@ -176,40 +189,6 @@ struct DevBuf {
   } while (0)
 
 size_t count_elem_size(int dtype) { return dtype == DEVIL_COUNTS_F64 ? 8 : 4; }
-
-// Host loops over cells split across threads ([lo, hi) ranges).
-template <typename F>
-void parallel_for(int64_t n, F&& fn) {
-  const int64_t hw = std::max<int64_t>(1, std::thread::hardware_concurrency());
-  const int64_t T = std::min<int64_t>({hw, 16, std::max<int64_t>(1, n / 65536)});
-  if (T <= 1) {
-    fn((int64_t)0, n);
-    return;
-  }
-  std::vector<std::thread> th;
-  th.reserve(T);
-  for (int64_t t = 0; t < T; ++t) th.emplace_back([&, t] { fn(n * t / T, n * (t + 1) / T); });
-  for (auto& x : th) x.join();
-}
-
-// Upper Cholesky factor of the p x p SPD matrix A (column-major): A = R'R.
-bool cholesky_upper(const double* A, int p, double* R) {
-  for (int j = 0; j < p; ++j)
-    for (int i = 0; i < p; ++i) R[i + j * p] = 0.0;
-  for (int j = 0; j < p; ++j) {
-    double d = A[j + j * p];
-    for (int k = 0; k < j; ++k) d -= R[k + j * p] * R[k + j * p];
-    if (!(d > 0.0)) return false;
-    const double r = std::sqrt(d);
-    R[j + j * p] = r;
-    for (int i = j + 1; i < p; ++i) {
-      double s = A[j + i * p];
-      for (int k = 0; k < j; ++k) s -= R[k + j * p] * R[k + i * p];
-      R[j + i * p] = s / r;
-    }
-  }
-  return true;
-}
 
 // Householder QR of the n x p column-major X: thin Q (n x p) and upper R.
 // Returns false when a diagonal of R is below 1e-7 of the largest, the rank
@@ -282,73 +261,73 @@ struct Design {
   int64_t n = 0;
   int p = 0;
   std::vector<double> X;  // host copy of X, made only when a host step needs it
-  std::vector<double> off, eo, logsf, R, xmean, denom;
-  double moi = 0.0, sum_sf = 0.0;
+  std::vector<double> eo, logsf, R, xmean, denom;
+  double sum_sf = 0.0;
   int intercept_first = 0;
 };
 
 // Device copies of the design, offsets and init operands.
 struct DeviceDesign {
-  DevBuf X, off, eo, Q, R, logsf, xmean, denom;
-  const double* x = nullptr;  // device X (the caller's own when it is device memory)
+  DevBuf X, offb, eo, moi, Q, R, logsf, xmean, denom;
+  // device X and offset (the caller's own where they are device memory)
+  const double* x = nullptr;
+  const double* off = nullptr;
+  bool qr = false;  // Q and R come from qr_device: finish_qr looks at its verdict
 };
 
-void combine_gram(const std::vector<double>& part, int p, std::vector<double>& G) {
-  G.assign((size_t)p * p, 0.0);
-  int q = 0;
-  for (int a = 0; a < p; ++a)
-    for (int b = a; b < p; ++b, ++q) {
-      long double su = 0.0L;
-      for (int x = 0; x < dv::kStatBlocksHost; ++x) su += part[x * 55 + q];
-      G[a + b * p] = G[b + a * p] = (double)su;
-    }
+// Pinned words that the set-up's kernels write: one wait serves them all.
+struct SetupHost {
+  uint64_t col[3 * dv::kMaxCand];  // launch_col_stats
+  int32_t differ[dv::kMaxPairs];   // launch_col_mismatch
+  int32_t qr_bad;                  // launch_chol
+};
+
+int setup_sync_setup(devil_ctx* ctx) {
+  if (ctx->setup_host) return DEVIL_OK;
+  void *h = nullptr, *d = nullptr;
+  DV_HIP(hipHostMalloc(&h, sizeof(SetupHost), hipHostMallocDefault));
+  ctx->setup_host = h;
+  DV_HIP(hipHostGetDevicePointer(&d, h, 0));
+  ctx->setup_dev = d;
+  return DEVIL_OK;
 }
 
 // Thin QR of the device X (n x p) by Cholesky QR applied twice on the GPU:
-// X'X = R1'R1, Q1 = X R1^-1, Q1'Q1 = R2'R2, Q = Q1 R2^-1, R = R2 R1.  ok is
-// false when a Gram matrix is not positive definite or a diagonal of R is
-// below 1e-7 of the largest (the rank tolerance of R's qr(), LINPACK dqrdc2).
-int qr_device(devil_ctx* ctx, const double* Xd, int64_t n, int p, DevBuf& Q,
-              std::vector<double>& R, bool& ok) {
+// X'X = R1'R1, Q1 = X R1^-1, Q1'Q1 = R2'R2, Q = Q1 R2^-1, R = R2 R1.  Nothing
+// is waited for; the verdict (a Gram matrix that is not positive definite, or a
+// diagonal of R below 1e-7 of the largest, the rank tolerance of R's qr(),
+// LINPACK dqrdc2) lands in SetupHost::qr_bad.
+int qr_device(devil_ctx* ctx, const double* Xd, int64_t n, int p, DevBuf& Q, DevBuf& R) {
   hipStream_t s = ctx->stream;
-  ok = false;
-  DV_ALLOC(Q, sizeof(double) * n * p);
-  DV_HIP(hipMemcpyAsync(Q.p, Xd, sizeof(double) * n * p, hipMemcpyDeviceToDevice, s));
-  DevBuf part, Rd;
-  DV_ALLOC(part, sizeof(double) * dv::kStatBlocksHost * 55);
-  DV_ALLOC(Rd, sizeof(double) * p * p);
-  std::vector<double> hp((size_t)dv::kStatBlocksHost * 55), G, R1((size_t)p * p),
-      R2((size_t)p * p);
-  auto gram = [&]() -> int {
-    DV_HIP(dv::launch_gram(s, Q.as<double>(), n, p, part.as<double>()));
-    DV_HIP(hipMemcpyAsync(hp.data(), part.p, sizeof(double) * hp.size(), hipMemcpyDeviceToHost,
-                          s));
-    DV_HIP(hipStreamSynchronize(s));
-    combine_gram(hp, p, G);
-    return DEVIL_OK;
-  };
   int rc;
-  if ((rc = gram())) return rc;
-  if (!cholesky_upper(G.data(), p, R1.data())) return DEVIL_OK;
-  DV_HIP(hipMemcpyAsync(Rd.p, R1.data(), sizeof(double) * p * p, hipMemcpyHostToDevice, s));
-  DV_HIP(dv::launch_right_solve(s, Q.as<double>(), n, p, Rd.as<double>()));
-  if ((rc = gram())) return rc;
-  if (!cholesky_upper(G.data(), p, R2.data())) return DEVIL_OK;
-  DV_HIP(hipMemcpyAsync(Rd.p, R2.data(), sizeof(double) * p * p, hipMemcpyHostToDevice, s));
-  DV_HIP(dv::launch_right_solve(s, Q.as<double>(), n, p, Rd.as<double>()));
-  DV_HIP(hipStreamSynchronize(s));
-  R.assign((size_t)p * p, 0.0);
-  for (int j = 0; j < p; ++j)
-    for (int i = 0; i <= j; ++i) {
-      double su = 0.0;
-      for (int k = i; k <= j; ++k) su += R2[i + k * p] * R1[k + j * p];
-      R[i + j * p] = su;
-    }
-  double dmax = 0.0;
-  for (int a = 0; a < p; ++a) dmax = std::max(dmax, std::fabs(R[a + a * p]));
-  ok = true;
-  for (int a = 0; a < p; ++a)
-    if (!(std::fabs(R[a + a * p]) > 1e-7 * dmax)) ok = false;
+  if ((rc = setup_sync_setup(ctx))) return rc;
+  int32_t* bad = &static_cast<SetupHost*>(ctx->setup_dev)->qr_bad;
+  DV_ALLOC(Q, sizeof(double) * n * p);
+  DV_ALLOC(R, sizeof(double) * p * p);
+  DV_HIP(hipMemcpyAsync(Q.p, Xd, sizeof(double) * n * p, hipMemcpyDeviceToDevice, s));
+  DevBuf part, R1, R2;
+  DV_ALLOC(part, sizeof(double) * dv::kStatBlocksHost * 55);
+  DV_ALLOC(R1, sizeof(double) * p * p);
+  DV_ALLOC(R2, sizeof(double) * p * p);
+  double* q = Q.as<double>();
+  DV_HIP(dv::launch_gram(s, q, n, p, part.as<double>()));
+  DV_HIP(dv::launch_chol(s, part.as<double>(), p, R1.as<double>(), nullptr, nullptr, bad));
+  DV_HIP(dv::launch_right_solve(s, q, n, p, R1.as<double>()));
+  DV_HIP(dv::launch_gram(s, q, n, p, part.as<double>()));
+  DV_HIP(dv::launch_chol(s, part.as<double>(), p, R1.as<double>(), R2.as<double>(),
+                         R.as<double>(), bad));
+  DV_HIP(dv::launch_right_solve(s, q, n, p, R2.as<double>()));
+  return DEVIL_OK;
+}
+
+// eo = exp(off) and moi = 1 / mean(eo) on the device.
+int exp_offsets(devil_ctx* ctx, const double* off, int64_t n, DevBuf& eo, DevBuf& moi) {
+  DevBuf part;
+  DV_ALLOC(eo, sizeof(double) * n);
+  DV_ALLOC(moi, sizeof(double));
+  DV_ALLOC(part, sizeof(double) * dv::kStatBlocksHost);
+  DV_HIP(dv::launch_exp_offsets(ctx->stream, off, n, eo.as<double>(), part.as<double>(),
+                                moi.as<double>()));
   return DEVIL_OK;
 }
 
@@ -362,48 +341,34 @@ int host_copy_of_x(devil_ctx* ctx, const double* X, int mem, Design& d) {
   return DEVIL_OK;
 }
 
-// Offsets, exp(offset) and the init operands on host and device; X stays on
-// the device (the caller's pointer when it is device memory).
+// Offsets, exp(offset) and the init operands on the device; X and the offsets
+// stay where they are when that is device memory.  Nothing is waited for (but
+// for the univariate start, which the host prepares).
 int prepare_design(devil_ctx* ctx, const double* X, const double* off, int64_t n, int p,
                    int mem, int init_mode, Design& d, DeviceDesign& dd) {
   d.n = n;
   d.p = p;
-  d.off.resize(n);
-  if (mem == DEVIL_MEM_DEVICE)
-    DV_HIP(hipMemcpy(d.off.data(), off, sizeof(double) * n, hipMemcpyDeviceToHost));
-  else
-    std::memcpy(d.off.data(), off, sizeof(double) * n);
-  d.eo.resize(n);
-  parallel_for(n, [&](int64_t lo, int64_t hi) {
-    for (int64_t i = lo; i < hi; ++i) d.eo[i] = std::exp(d.off[i]);  // exp_offset, R/main.R:390
-  });
-  double se = 0.0;
-  for (int64_t i = 0; i < n; ++i) se += d.eo[i];
-  d.moi = 1.0 / (se / (double)n);  // R/overdispersion.R:130
+  hipStream_t s = ctx->stream;
   int rc;
   if (mem == DEVIL_MEM_DEVICE) {
     dd.x = X;
+    dd.off = off;
   } else {
     if ((rc = upload_raw(ctx, dd.X, X, sizeof(double) * n * p, hipMemcpyHostToDevice))) return rc;
+    if ((rc = upload_raw(ctx, dd.offb, off, sizeof(double) * n, hipMemcpyHostToDevice))) return rc;
     dd.x = dd.X.as<double>();
+    dd.off = dd.offb.as<double>();
   }
-  if ((rc = upload(ctx, dd.off, d.off))) return rc;
-  if ((rc = upload(ctx, dd.eo, d.eo))) return rc;
+  if ((rc = exp_offsets(ctx, dd.off, n, dd.eo, dd.moi))) return rc;
   if (init_mode == DEVIL_INIT_QR) {
-    bool ok = false;
-    if ((rc = qr_device(ctx, dd.x, n, p, dd.Q, d.R, ok))) return rc;
-    if (!ok) {  // ill-conditioned for Cholesky QR: Householder on the host
-      if ((rc = host_copy_of_x(ctx, X, mem, d))) return rc;
-      std::vector<double> Qh;
-      if (!householder_qr(d.X.data(), n, p, Qh, d.R))
-        return fail(ctx, DEVIL_E_RANK, "design matrix is rank deficient (QR init, R/beta.R:14)");
-      if ((rc = upload(ctx, dd.Q, Qh))) return rc;
-      DV_HIP(hipStreamSynchronize(ctx->stream));
-    }
-    if ((rc = upload(ctx, dd.R, d.R))) return rc;
+    if ((rc = qr_device(ctx, dd.x, n, p, dd.Q, dd.R))) return rc;
+    dd.qr = true;
   } else if (init_mode == DEVIL_INIT_UNIVARIATE) {
     // src/beta_init_univariate.cpp:48-84
     if ((rc = host_copy_of_x(ctx, X, mem, d))) return rc;
+    d.eo.resize(n);
+    DV_HIP(hipMemcpyAsync(d.eo.data(), dd.eo.p, sizeof(double) * n, hipMemcpyDeviceToHost, s));
+    DV_HIP(hipStreamSynchronize(s));
     double mx = 0.0;
     for (int64_t i = 0; i < n; ++i) mx = std::max(mx, std::fabs(d.X[i] - 1.0));
     d.intercept_first = mx < 1e-10;
@@ -430,6 +395,21 @@ int prepare_design(devil_ctx* ctx, const double* X, const double* off, int64_t n
     if ((rc = upload(ctx, dd.xmean, d.xmean))) return rc;
     if ((rc = upload(ctx, dd.denom, d.denom))) return rc;
   }
+  return DEVIL_OK;
+}
+
+// The verdict of qr_device, once the stream has been synchronised: a design
+// too ill-conditioned for Cholesky QR gets its Householder QR on the host.
+int finish_qr(devil_ctx* ctx, const double* X, int mem, Design& d, DeviceDesign& dd) {
+  if (!dd.qr || !static_cast<const volatile SetupHost*>(ctx->setup_host)->qr_bad) return DEVIL_OK;
+  int rc;
+  if ((rc = host_copy_of_x(ctx, X, mem, d))) return rc;
+  std::vector<double> Qh;
+  if (!householder_qr(d.X.data(), d.n, d.p, Qh, d.R))
+    return fail(ctx, DEVIL_E_RANK, "design matrix is rank deficient (QR init, R/beta.R:14)");
+  if ((rc = upload(ctx, dd.Q, Qh))) return rc;
+  if ((rc = upload(ctx, dd.R, d.R))) return rc;
+  DV_HIP(hipStreamSynchronize(ctx->stream));
   return DEVIL_OK;
 }
 
@@ -556,56 +536,71 @@ struct ColPlan {
   int kidx_lin[10];
 };
 
-// Statistics of every candidate column computed on the device (Xd: device
-// n x p X); equal hashes are confirmed by a cell-by-cell comparison.
-int plan_columns(devil_ctx* ctx, const double* Xd, int64_t n, int p, bool lin16, ColPlan& cp) {
-  hipStream_t s = ctx->stream;
+// Statistics of every candidate column of a design, and which of them are
+// equal: equal hashes are confirmed by a cell-by-cell comparison.  Two waits
+// for the device (one where no two candidates have the same hash).
+struct ColStats {
   std::vector<dv::ColSpec> cand;
-  for (int a = 0; a < p; ++a) cand.push_back({a, -1});
+  std::vector<uint64_t> hash, nonzero;
+  std::vector<double> sum;
+  std::vector<char> differ;  // C x C, for pairs of one hash
+};
+
+int column_stats(devil_ctx* ctx, const double* Xd, int64_t n, int p, ColStats& cs) {
+  hipStream_t s = ctx->stream;
+  for (int a = 0; a < p; ++a) cs.cand.push_back({a, -1});
   for (int a = 0; a < p; ++a)
-    for (int b = a; b < p; ++b) cand.push_back({a, b});
-  const int C = (int)cand.size();
-  const int B = dv::kStatBlocksHost;
-  DevBuf dc, dh, dnz, dsum, dmm;
+    for (int b = a; b < p; ++b) cs.cand.push_back({a, b});
+  const int C = (int)cs.cand.size();
   int rc;
-  if ((rc = upload(ctx, dc, cand))) return rc;
-  DV_ALLOC(dh, sizeof(uint64_t) * C * B);
-  DV_ALLOC(dnz, sizeof(uint64_t) * C * B);
-  DV_ALLOC(dsum, sizeof(double) * C * B);
-  DV_ALLOC(dmm, sizeof(uint64_t) * B);
-  DV_HIP(dv::launch_col_stats(s, Xd, n, dc.as<dv::ColSpec>(), C, dh.as<uint64_t>(),
-                              dnz.as<uint64_t>(), dsum.as<double>()));
-  std::vector<uint64_t> ph((size_t)C * B), pnz((size_t)C * B);
-  std::vector<double> psum((size_t)C * B);
-  DV_HIP(hipMemcpyAsync(ph.data(), dh.p, sizeof(uint64_t) * C * B, hipMemcpyDeviceToHost, s));
-  DV_HIP(hipMemcpyAsync(pnz.data(), dnz.p, sizeof(uint64_t) * C * B, hipMemcpyDeviceToHost, s));
-  DV_HIP(hipMemcpyAsync(psum.data(), dsum.p, sizeof(double) * C * B, hipMemcpyDeviceToHost, s));
+  if ((rc = setup_sync_setup(ctx))) return rc;
+  SetupHost* h = static_cast<SetupHost*>(ctx->setup_host);
+  SetupHost* d = static_cast<SetupHost*>(ctx->setup_dev);
+  DevBuf part;
+  DV_ALLOC(part, sizeof(uint64_t) * 3 * C * dv::kStatBlocksHost);
+  DV_HIP(dv::launch_col_stats(s, Xd, n, p, part.as<uint64_t>(), d->col));
   DV_HIP(hipStreamSynchronize(s));
-  std::vector<uint64_t> hash(C, 0), nonzero(C, 0);
-  std::vector<double> sum(C, 0.0);
+  cs.hash.resize(C);
+  cs.nonzero.resize(C);
+  cs.sum.resize(C);
   for (int c = 0; c < C; ++c) {
-    long double su = 0.0L;
-    for (int x = 0; x < B; ++x) {
-      hash[c] += ph[(size_t)c * B + x];
-      nonzero[c] += pnz[(size_t)c * B + x];
-      su += psum[(size_t)c * B + x];
-    }
-    sum[c] = (double)su;
+    cs.hash[c] = h->col[3 * c];
+    cs.nonzero[c] = h->col[3 * c + 1];
+    std::memcpy(&cs.sum[c], &h->col[3 * c + 2], sizeof(double));
   }
-  std::vector<int> members;  // candidate behind each column (-1: padding)
-  std::vector<uint64_t> mm(B);
-  int err = DEVIL_OK;
-  auto equal = [&](int c1, int c2) -> bool {
-    if (dv::launch_col_mismatch(s, Xd, n, cand[c1], cand[c2], dmm.as<uint64_t>()) != hipSuccess ||
-        hipMemcpyAsync(mm.data(), dmm.p, sizeof(uint64_t) * B, hipMemcpyDeviceToHost, s) !=
-            hipSuccess ||
-        hipStreamSynchronize(s) != hipSuccess) {
-      err = fail(ctx, DEVIL_E_HIP, "column comparison failed");
-      return false;
+  cs.differ.assign((size_t)C * C, 1);
+  dv::ColPairs pairs;
+  std::vector<int> at;
+  pairs.n = 0;
+  auto flush = [&]() -> int {
+    if (pairs.n == 0) return DEVIL_OK;
+    std::memset(h->differ, 0, sizeof(h->differ));
+    DV_HIP(dv::launch_col_mismatch(s, Xd, n, pairs, d->differ));
+    DV_HIP(hipStreamSynchronize(s));
+    for (int q = 0; q < pairs.n; ++q) cs.differ[at[q]] = h->differ[q] != 0;
+    pairs.n = 0;
+    at.clear();
+    return DEVIL_OK;
+  };
+  for (int c1 = 0; c1 < C; ++c1)
+    for (int c2 = c1 + 1; c2 < C; ++c2) {
+      if (!cs.nonzero[c1] || !cs.nonzero[c2] || cs.hash[c1] != cs.hash[c2]) continue;
+      pairs.c1[pairs.n] = cs.cand[c1];
+      pairs.c2[pairs.n++] = cs.cand[c2];
+      at.push_back(c1 * C + c2);
+      if (pairs.n == dv::kMaxPairs && (rc = flush())) return rc;
     }
-    uint64_t tot = 0;
-    for (uint64_t v : mm) tot += v;
-    return tot == 0;
+  return flush();
+}
+
+void plan_columns(const ColStats& cs, int p, bool lin16, ColPlan& cp) {
+  const std::vector<dv::ColSpec>& cand = cs.cand;
+  const std::vector<uint64_t>&hash = cs.hash, &nonzero = cs.nonzero;
+  const std::vector<double>& sum = cs.sum;
+  const int C = (int)cand.size();
+  std::vector<int> members;  // candidate behind each column (-1: padding)
+  auto equal = [&](int c1, int c2) {
+    return !cs.differ[std::min(c1, c2) * C + std::max(c1, c2)];
   };
   auto add = [&](int c) -> int {
     if (!nonzero[c]) return -1;
@@ -632,7 +627,13 @@ int plan_columns(devil_ctx* ctx, const double* Xd, int64_t n, int p, bool lin16,
     for (int a = 0; a < p; ++a) cp.kidx_lin[a] = add(a);
   }
   for (int q = 0; q < p * (p + 1) / 2; ++q) cp.kidx_pair[q] = add(p + q);
-  return err;
+}
+
+dv::ColList col_list(const ColPlan& cp) {
+  dv::ColList l;
+  l.n = (int)std::min<size_t>(cp.spec.size(), DEVIL_NCP_MAX);
+  for (int c = 0; c < l.n; ++c) l.c[c] = cp.spec[c];
+  return l;
 }
 
 // Chunks of about chunk_blocks blocks.  Chunk boundaries fall on multiples of
@@ -681,7 +682,7 @@ struct TileHost {
   const double* off = nullptr;  // device offsets
   int intercept = 0;            // column 0 of X is all ones
   int mixed = kMixedNone;
-  DevBuf spec, specm, Xp, offp, eop, Kp, Xf, offf, Kf, xab, offl, kg, kh, kh2;
+  DevBuf Xp, offp, eop, Kp, Xf, offf, Kf, xab, offl, kg, kh, kh2;
 };
 
 // The FP64 IRLS takes one workgroup per gene where the design stays in an
@@ -699,12 +700,13 @@ int make_tile(devil_ctx* ctx, const double* Xd, const double* offd, const double
   th.mixed = mixed;
   th.X = Xd;
   th.off = offd;
+  ColStats cs;
   ColPlan cp;
   int rc;
-  if ((rc = plan_columns(ctx, Xd, n, p, false, cp))) return rc;
+  if ((rc = column_stats(ctx, Xd, n, p, cs))) return rc;
+  plan_columns(cs, p, false, cp);
   dv::TileDesign& td = th.td;
   shape_design(cp, n, p, 16, td, chunk_cells);
-  if ((rc = upload(ctx, th.spec, cp.spec))) return rc;
   const int NJ = (p + 3) / 4;
   DV_ALLOC(th.Xp, sizeof(double) * td.nblk * NJ * 64);
   DV_ALLOC(th.offp, sizeof(double) * td.nblk * 16);
@@ -716,8 +718,8 @@ int make_tile(devil_ctx* ctx, const double* Xd, const double* offd, const double
     DV_ALLOC(th.offf, sizeof(float) * td.nblk * 16);
     DV_ALLOC(th.Kf, sizeof(float) * td.nblk * td.nt * 256);
   }
-  DV_HIP(dv::launch_build_tables(s, Xd, offd, eod, n, p, th.spec.as<dv::ColSpec>(),
-                                 (int)cp.spec.size(), td.nt, td.nblk, th.Xp.as<double>(),
+  DV_HIP(dv::launch_build_tables(s, Xd, offd, eod, n, p, col_list(cp), td.nt, td.nblk,
+                                 th.Xp.as<double>(),
                                  th.offp.as<double>(), th.eop.as<double>(), th.Kp.as<double>(),
                                  f32 ? 1 : 0, th.Xf.as<float>(), th.offf.as<float>(),
                                  th.Kf.as<float>()));
@@ -737,10 +739,9 @@ int make_tile(devil_ctx* ctx, const double* Xd, const double* offd, const double
     th.tdm.Kf = th.Kf.as<float>();
   } else if (bf16_layout(mixed)) {
     ColPlan cm;
-    if ((rc = plan_columns(ctx, Xd, n, p, true, cm))) return rc;
+    plan_columns(cs, p, true, cm);
     dv::TileDesign& tm = th.tdm;
     shape_design(cm, n, p, 32, tm, chunk_cells);
-    if ((rc = upload(ctx, th.specm, cm.spec))) return rc;
     const int64_t nst = tm.nblk;
     const int NE = dv::eta_blocks(p);
     const int nth = tm.nt - 1;
@@ -757,8 +758,8 @@ int make_tile(devil_ctx* ctx, const double* Xd, const double* offd, const double
       DV_HIP(dv::launch_fill_i32(s, reinterpret_cast<int32_t*>(th.kh.p), words, 0));
       DV_HIP(dv::launch_fill_i32(s, reinterpret_cast<int32_t*>(th.kh2.p), words, 0));
     }
-    DV_HIP(dv::launch_build_tables_bf16(s, Xd, offd, n, p, th.specm.as<dv::ColSpec>(),
-                                        (int)cm.spec.size(), nth, nst, th.xab.as<uint16_t>(),
+    DV_HIP(dv::launch_build_tables_bf16(s, Xd, offd, n, p, col_list(cm), nth, nst,
+                                        th.xab.as<uint16_t>(),
                                         th.offl.as<float>(), th.kg.as<uint16_t>(),
                                         th.kh.as<uint16_t>(), th.kh2.as<uint16_t>()));
     tm.xab = th.xab.as<uint16_t>();
@@ -785,7 +786,7 @@ int build_init_tile(devil_ctx* ctx, const Design& d, const DeviceDesign& dd,
   const int p = d.p;
   dv::InitTile& it = ih.it;
   it.want_alpha = want_alpha;
-  it.moi = d.moi;
+  it.moi = dd.moi.as<double>();
   it.mode = mode;
   it.intercept_first = d.intercept_first;
   it.sum_sf = d.sum_sf;
@@ -810,16 +811,10 @@ int build_init_tile(devil_ctx* ctx, const Design& d, const DeviceDesign& dd,
 // FP64 tile design from a device-resident design matrix and offset.
 int tile_from_device(devil_ctx* ctx, const double* X, const double* offset, int64_t n, int p,
                      TileHost& th, int mixed = kMixedNone) {
-  std::vector<double> eo(n);
-  DV_HIP(hipMemcpy(eo.data(), offset, sizeof(double) * n, hipMemcpyDeviceToHost));
-  parallel_for(n, [&](int64_t lo, int64_t hi) {
-    for (int64_t i = lo; i < hi; ++i) eo[i] = std::exp(eo[i]);
-  });
-  DevBuf eod;
+  DevBuf eod, moi;
   int rc;
-  if ((rc = upload(ctx, eod, eo))) return rc;
+  if ((rc = exp_offsets(ctx, offset, n, eod, moi))) return rc;
   if ((rc = make_tile(ctx, X, offset, eod.as<double>(), n, p, mixed, th))) return rc;
-  DV_HIP(hipStreamSynchronize(ctx->stream));  // eod is freed on return
   return DEVIL_OK;
 }
 
@@ -835,9 +830,9 @@ int tile_from_device(devil_ctx* ctx, const double* X, const double* offset, int6
 constexpr int64_t kPostWaves = 4096;
 
 struct ChunkHost {
-  std::vector<int64_t> c0, c1;
+  std::vector<int64_t> c0, c1, all;
   std::vector<int32_t> cl;
-  DevBuf d0, d1, dcl;
+  DevBuf d;
   dv::ChunkTable ct{};
 };
 
@@ -879,14 +874,18 @@ int build_chunks(devil_ctx* ctx, int64_t n, const int32_t* ends, int C, int64_t 
       ch.c1.push_back(n);
       ch.cl.push_back(nc - 1);
     }
+  // [c0 | c1 | cl] in one transfer
+  const size_t m = ch.c0.size();
+  ch.all.resize(2 * m + (m + 1) / 2);
+  std::memcpy(ch.all.data(), ch.c0.data(), sizeof(int64_t) * m);
+  std::memcpy(ch.all.data() + m, ch.c1.data(), sizeof(int64_t) * m);
+  std::memcpy(ch.all.data() + 2 * m, ch.cl.data(), sizeof(int32_t) * m);
   int rc;
-  if ((rc = upload(ctx, ch.d0, ch.c0))) return rc;
-  if ((rc = upload(ctx, ch.d1, ch.c1))) return rc;
-  if ((rc = upload(ctx, ch.dcl, ch.cl))) return rc;
-  ch.ct.c0 = ch.d0.as<int64_t>();
-  ch.ct.c1 = ch.d1.as<int64_t>();
-  ch.ct.cl = ch.dcl.as<int32_t>();
-  ch.ct.nchunk = (int)ch.c0.size();
+  if ((rc = upload(ctx, ch.d, ch.all))) return rc;
+  ch.ct.c0 = ch.d.as<int64_t>();
+  ch.ct.c1 = ch.d.as<int64_t>() + m;
+  ch.ct.cl = reinterpret_cast<const int32_t*>(ch.d.as<int64_t>() + 2 * m);
+  ch.ct.nchunk = (int)m;
   return DEVIL_OK;
 }
 
@@ -1671,7 +1670,7 @@ int autotune_mixed(devil_ctx* ctx, const DeviceDesign& dd, int64_t n, int p, dv:
   for (int kind : kinds)
     for (int64_t cl : cells) {
       TileHost th;
-      if ((rc = make_tile(ctx, dd.x, dd.off.as<double>(), dd.eo.as<double>(), n, p, kind, th, cl)))
+      if ((rc = make_tile(ctx, dd.x, dd.off, dd.eo.as<double>(), n, p, kind, th, cl)))
         break;
       const dv::TileDesign& tm = th.tdm;
       DevBuf part;
@@ -1794,6 +1793,7 @@ void devil_destroy(devil_ctx* ctx) {
   for (hipEvent_t e : ctx->round_ev)
     if (e) (void)hipEventDestroy(e);
   if (ctx->round_counts) (void)hipHostFree(ctx->round_counts);
+  if (ctx->setup_host) (void)hipHostFree(ctx->setup_host);
   if (ctx->joint_host) (void)hipHostFree(ctx->joint_host);
   if (ctx->pad_p) (void)hipFree(ctx->pad_p);
   ctx->cache.clear();
@@ -1896,21 +1896,30 @@ int run_setup(devil_ctx* ctx, const devil_problem* pr, devil_outputs* out, ProbR
     if (ctx->tune[DEVIL_TUNE_CHUNK_CELLS] == 0) r.cc = (int64_t)(v >> 8);
     r.autotune = false;
   }
-  if ((rc = make_tile(ctx, r.dd.x, r.dd.off.as<double>(), r.dd.eo.as<double>(), n, p,
+  if ((rc = make_tile(ctx, r.dd.x, r.dd.off, r.dd.eo.as<double>(), n, p,
                       r.autotune ? kMixedNone : r.mk, r.tl, r.cc)))
     return rc;
+  if ((rc = finish_qr(ctx, pr->X, mem, r.d, r.dd))) return rc;
 
-  // per-gene device state (gene-major)
+  // per-gene device state (gene-major); what leaves as it is goes straight to
+  // the caller's device memory
+  const bool dev_out = mem == DEVIL_MEM_DEVICE;
   DV_ALLOC(r.alpha0, sizeof(double) * G);
   DV_ALLOC(r.kvec, sizeof(double) * G);
   DV_ALLOC(r.beta, sizeof(double) * G * p);
-  DV_ALLOC(r.theta, sizeof(double) * G);
-  DV_ALLOC(r.iters, sizeof(int32_t) * G);
-  DV_ALLOC(r.thit, sizeof(int32_t) * G);
-  DV_ALLOC(r.status, sizeof(int32_t) * G);
-  DV_ALLOC(r.bread, sizeof(double) * G * p * p);
+  if (dev_out) r.theta.borrow(out->theta);
+  else DV_ALLOC(r.theta, sizeof(double) * G);
+  if (dev_out) r.iters.borrow(out->beta_iters);
+  else DV_ALLOC(r.iters, sizeof(int32_t) * G);
+  if (dev_out) r.thit.borrow(out->theta_iters);
+  else DV_ALLOC(r.thit, sizeof(int32_t) * G);
+  if (dev_out && out->status) r.status.borrow(out->status);
+  else DV_ALLOC(r.status, sizeof(int32_t) * G);
+  if (dev_out) r.bread.borrow(out->bread);
+  else DV_ALLOC(r.bread, sizeof(double) * G * p * p);
   r.want_sw = C > 0 && out->sandwich;
-  if (r.want_sw) DV_ALLOC(r.sandwich, sizeof(double) * G * p * p);
+  if (r.want_sw && dev_out) r.sandwich.borrow(out->sandwich);
+  else if (r.want_sw) DV_ALLOC(r.sandwich, sizeof(double) * G * p * p);
 
   hipStream_t s = ctx->stream;
   if (pr->disp_init) {
@@ -2029,7 +2038,7 @@ int run_batch_init(devil_ctx* ctx, ProbRun& r, int64_t g0, StageTimer& tm) {
     ctx->tuned[r.key] = r.mk | (int)(r.cc << 8);
     r.autotune = false;
     r.tl = TileHost();
-    if ((rc = make_tile(ctx, r.dd.x, r.dd.off.as<double>(), r.dd.eo.as<double>(), r.n, r.p, r.mk,
+    if ((rc = make_tile(ctx, r.dd.x, r.dd.off, r.dd.eo.as<double>(), r.n, r.p, r.mk,
                         r.tl, r.cc)))
       return rc;
   }
@@ -2108,11 +2117,15 @@ int run_outputs(devil_ctx* ctx, ProbRun& r) {
   hipStream_t s = ctx->stream;
   const int64_t G = r.G;
   const int p = r.p;
+  if (pr->mem == DEVIL_MEM_DEVICE) {  // the rest is there already
+    DV_HIP(dv::launch_transpose_gp(s, r.beta.as<double>(), G, p, 0, out->beta));
+    DV_HIP(hipStreamSynchronize(s));
+    return DEVIL_OK;
+  }
   DevBuf bcol;
   DV_ALLOC(bcol, sizeof(double) * G * p);
   DV_HIP(dv::launch_transpose_gp(s, r.beta.as<double>(), G, p, 0, bcol.as<double>()));
-  const hipMemcpyKind kind =
-      pr->mem == DEVIL_MEM_DEVICE ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost;
+  const hipMemcpyKind kind = hipMemcpyDeviceToHost;
   DV_HIP(hipMemcpyAsync(out->beta, bcol.p, sizeof(double) * G * p, kind, s));
   DV_HIP(hipMemcpyAsync(out->theta, r.theta.p, sizeof(double) * G, kind, s));
   DV_HIP(hipMemcpyAsync(out->beta_iters, r.iters.p, sizeof(int32_t) * G, kind, s));
@@ -2932,22 +2945,15 @@ int devil_estimate_dispersion(devil_ctx* ctx, const void* counts, int32_t dtype,
   if ((rc = set_device(ctx))) return rc;
   if ((rc = check_counts_args(ctx, counts, dtype, G, n, ld))) return rc;
   if (!offset || (G > 0 && !alpha0)) return fail(ctx, DEVIL_E_ARG, "NULL pointer");
-  std::vector<double> off(n);
-  DV_HIP(hipMemcpy(off.data(), offset, sizeof(double) * n, hipMemcpyDeviceToHost));
-  double se = 0.0;
-  for (int64_t i = 0; i < n; ++i) se += std::exp(off[i]);
   if (G == 0) return DEVIL_OK;
   Design d;
   d.n = n;
   d.p = 1;
-  d.moi = 1.0 / (se / (double)n);
-  d.eo.resize(n);
-  for (int64_t i = 0; i < n; ++i) d.eo[i] = std::exp(off[i]);
   dv::TileDesign td{};
   td.n = n;
   td.nblk = (n + 15) / 16;
   DeviceDesign dd;
-  if ((rc = upload(ctx, dd.eo, d.eo))) return rc;
+  if ((rc = exp_offsets(ctx, offset, n, dd.eo, dd.moi))) return rc;
   InitHost ih;
   if ((rc = build_init_tile(ctx, d, dd, td, 1, dv::kInitNone, ih))) return rc;
   ChunkHost chunks;
@@ -2974,6 +2980,8 @@ int devil_init_beta(devil_ctx* ctx, const void* counts, int32_t dtype, int64_t G
   Design d;
   DeviceDesign dd;
   if ((rc = prepare_design(ctx, X, offset, n, p, DEVIL_MEM_DEVICE, init_mode, d, dd))) return rc;
+  DV_HIP(hipStreamSynchronize(ctx->stream));
+  if ((rc = finish_qr(ctx, X, DEVIL_MEM_DEVICE, d, dd))) return rc;
   if (G == 0) return DEVIL_OK;
   dv::TileDesign td{};
   td.n = n;

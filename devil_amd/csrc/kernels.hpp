@@ -64,23 +64,48 @@ struct TileDesign {
 struct ColSpec {
   int a, b;
 };
+// The columns of K, passed to the table kernels by value.
+struct ColList {
+  int n;
+  ColSpec c[DEVIL_NCP_MAX];
+};
 hipError_t launch_build_tables(hipStream_t s, const double* X, const double* off,
-                               const double* eo, int64_t n, int p, const ColSpec* spec, int ncol,
-                               int nt, int64_t nblk, double* Xp, double* offp, double* eop,
-                               double* Kp, int f32, float* Xf, float* offf, float* Kf);
+                               const double* eo, int64_t n, int p, const ColList& cols, int nt,
+                               int64_t nblk, double* Xp, double* offp, double* eop, double* Kp,
+                               int f32, float* Xf, float* offf, float* Kf);
 // Design statistics on the device: partials per kStatBlocks cell ranges.
 constexpr int kStatBlocksHost = 64;
-hipError_t launch_col_stats(hipStream_t s, const double* X, int64_t n, const ColSpec* cand,
-                            int C, uint64_t* ph, uint64_t* pnz, double* ps);
-hipError_t launch_col_mismatch(hipStream_t s, const double* X, int64_t n, ColSpec c1, ColSpec c2,
-                               uint64_t* out);
+constexpr int kMaxCand = 65;  // p design columns and p (p + 1) / 2 products
+// Statistics of every candidate column, in the order of the design columns
+// and the products (a <= b): out[3 c + 0 .. 2] = order-free hash, non-zero
+// cells, sum (as a double's bits); part holds 3 C kStatBlocksHost words.
+hipError_t launch_col_stats(hipStream_t s, const double* X, int64_t n, int p, uint64_t* part,
+                            uint64_t* out);
+// out[q] = 1 where the q-th pair of candidates differs in some cell (out is
+// cleared by the caller).
+constexpr int kMaxPairs = 64;
+struct ColPairs {
+  int n;
+  ColSpec c1[kMaxPairs], c2[kMaxPairs];
+};
+hipError_t launch_col_mismatch(hipStream_t s, const double* X, int64_t n, const ColPairs& pairs,
+                               int32_t* out);
+// eo = exp(off) and *moi = 1 / mean(eo); part: kStatBlocksHost doubles.
+hipError_t launch_exp_offsets(hipStream_t s, const double* off, int64_t n, double* eo,
+                              double* part, double* moi);
 hipError_t launch_gram(hipStream_t s, const double* M, int64_t n, int p, double* out);  // [64][55]
+// Upper Cholesky factor (column-major) of the Gram matrix whose partials are
+// part: first of the design (out1), then of its orthogonalised columns, when
+// out = (the second factor) out1 is the R of the design.  *bad is set where a
+// pivot is not positive, or a diagonal of R below 1e-7 of the largest.
+hipError_t launch_chol(hipStream_t s, const double* part, int p, double* out1, double* out2,
+                       double* out, int32_t* bad);
 hipError_t launch_right_solve(hipStream_t s, double* M, int64_t n, int p, const double* R);
 hipError_t launch_build_init(hipStream_t s, const double* M, const double* shift,
                              const double* eo, const double* logsf, int64_t n, int p,
                              int64_t nblk, double* Zp, double* einv, double* logsfp);
 hipError_t launch_build_tables_bf16(hipStream_t s, const double* X, const double* off, int64_t n,
-                                    int p, const ColSpec* spec, int ncol, int nth, int64_t nst,
+                                    int p, const ColList& cols, int nth, int64_t nst,
                                     uint16_t* xab, float* offl, uint16_t* kg, uint16_t* kh,
                                     uint16_t* kh2);
 
@@ -98,7 +123,7 @@ struct ChunkTable {
 // one 16-column tile, [blk][lane][r] = Z[16 blk + 4 (lane/16) + r][lane%16].
 struct InitTile {
   int want_alpha;
-  double moi;            // 1 / mean(exp(offset))
+  const double* moi;     // 1 / mean(exp(offset)), on the device
   int mode;              // kInit*
   const double* Zp;      // projection columns (QR: thin Q; univariate: X - mean)
   const double* einv;    // exp(-offset), padded to 16 nblk

@@ -592,7 +592,7 @@ __global__ __launch_bounds__(256) void k_init_finish(InitTile it, ChunkTable ct,
   const double mean = s1 / (double)n;
   if (it.want_alpha) {
     const double v = ssd / (double)(n - 1);
-    const double d = (v - it.moi * mean) / (mean * mean);
+    const double d = (v - *it.moi * mean) / (mean * mean);
     alpha0[g] = (isnan(d) || d < 0.0) ? 0.01 : d;
   }
   if (it.mode == kInitNone) return;

@@ -89,3 +89,30 @@ def test_round_kernels(dv, orc, G, p, intercept):
     active genes, 16-gene tiles above."""
     Y, X, sf = problem(G, (2 << 20) // (8 * (p + 1)) + 77, p, intercept)
     check(dv, orc, Y, X, sf)
+
+
+def test_design_setup(dv, orc):
+    """The design's QR and its equal columns, found on the device: all nine
+    indicators of a factor beside an intercept are rank deficient; with eight of
+    them (54 candidates, many equal or zero), with products among the columns
+    and with nearly collinear columns the fit is the oracle's."""
+    r = np.random.default_rng(5)
+    n, G = 4000, 20
+    lv = r.integers(0, 9, n)
+    X = np.column_stack([np.ones(n)] + [lv == k for k in range(9)]).astype(float)
+    Y = r.poisson(np.exp(0.5 + 0.1 * lv) * r.gamma(2.0, 0.5, (G, n))).astype(np.int32)
+    sf = np.exp(r.normal(0, 0.2, n))
+    with pytest.raises(Exception, match="rank deficient"):
+        dv.fit_devil(torch.as_tensor(Y, device="cuda"), X, size_factors=sf)
+    check(dv, orc, Y, np.ascontiguousarray(X[:, :9]), sf)
+    g = (lv > 4).astype(float)
+    h = (lv % 2).astype(float)
+    Xd = np.column_stack([np.ones(n), g, h, g * h])
+    check(dv, orc, Y, Xd, sf)
+    z = r.normal(size=n)
+    Xc = np.column_stack([np.ones(n), z, z + 1e-3 * r.normal(size=n)])
+    fit = dv.fit_devil(torch.as_tensor(Y, device="cuda"), Xc, size_factors=sf,
+                       overdispersion=False)
+    ref = orc.cpu_fit(Y.astype(np.float64), Xc, np.log(sf), od_mode=orc.OD_NONE)
+    # the condition number 2e3 enters the normal equations squared: 4e6 * 2^-53
+    np.testing.assert_allclose(fit["beta"].cpu().numpy(), ref["beta"], rtol=1e-8, atol=1e-8)
