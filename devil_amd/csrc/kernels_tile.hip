@@ -43,6 +43,7 @@
 #include "irls_tile.hpp"
 #include "kernels.hpp"
 #include "tile_common.hpp"
+#include "wave_solve.hpp"
 
 namespace dv {
 
@@ -1201,24 +1202,42 @@ __device__ __forceinline__ void irls_update_body(const TileDesign& td, int i,
   __syncthreads();
   if (lane >= 64) return;
   const double k = kvec[g];
-  double M[P][P], v[P];
+  double v[P];
+  int sing;
+  // up to p = 2 one lane's LU is the shorter; above, a row per lane (p = 8: the
+  // update of a round of few genes 10 -> 6 us)
+  if constexpr (P <= 2) {
+    double M[P][P];
 #pragma unroll
-  for (int a = 0; a < P; ++a) {
-    const int gi = td.kidx_lin[a];
-    v[a] = k * (gi >= 0 ? acc[gi] : 0.0);
+    for (int a = 0; a < P; ++a) {
+      const int gi = td.kidx_lin[a];
+      v[a] = k * (gi >= 0 ? acc[gi] : 0.0);
 #pragma unroll
-    for (int bb = a; bb < P; ++bb) {
-      const int pi = td.kidx_pair[tri<P>(a, bb)];
-      const double e = k * (pi >= 0 ? acc[pi] + td.ksum[pi] : 0.0);
-      M[a][bb] = e;
-      M[bb][a] = e;
+      for (int bb = a; bb < P; ++bb) {
+        const int pi = td.kidx_pair[tri<P>(a, bb)];
+        const double e = k * (pi >= 0 ? acc[pi] + td.ksum[pi] : 0.0);
+        M[a][bb] = e;
+        M[bb][a] = e;
+      }
     }
+    int perm[P];
+    sing = lu_factor<P>(M, perm);
+    lu_solve<P>(M, perm, v);
+  } else {
+    const int li = min(lane, P - 1);
+    double row[P];
+#pragma unroll
+    for (int j = 0; j < P; ++j) {
+      const int a = min(li, j), c = max(li, j);
+      const int pi = td.kidx_pair[a * P - a * (a - 1) / 2 + (c - a)];
+      row[j] = k * (pi >= 0 ? acc[pi] + td.ksum[pi] : 0.0);
+    }
+    const int gi = td.kidx_lin[li];
+    sing = wave_lu_solve<P>(row, k * (gi >= 0 ? acc[gi] : 0.0), lane, v);
   }
   if (lane != 0) return;
   int st = status[g];
-  int perm[P];
-  if (lu_factor<P>(M, perm)) st |= DEVIL_GENE_SINGULAR;
-  lu_solve<P>(M, perm, v);
+  if (sing) st |= DEVIL_GENE_SINGULAR;
   double mx = 0.0;
   bool has_nan = false;
 #pragma unroll
