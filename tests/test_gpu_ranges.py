@@ -116,3 +116,22 @@ def test_vector_columns(dv, orc, extra, patients):
             m = orc.meat_hc0(X, Y[g].astype(float), b[g], th[g], sf)
             want.append(h @ m @ h * n)
         close(sw[::13], np.array(want), "HC0")
+
+
+@pytest.mark.parametrize("dtype", [np.int32, np.float32, np.float64])
+def test_init_large_counts(dv, orc, dtype):
+    """Counts on both sides of 2^14 in one block, and zeros: the init pass takes
+    its short form only for whole blocks below."""
+    r = np.random.default_rng(3)
+    G, n = 40, 2100
+    X = np.column_stack([np.ones(n), r.normal(size=n)])
+    sf = np.exp(r.normal(0, 0.3, n))
+    Y = r.poisson(sf * r.gamma(3.0, 2.0, (G, n))).astype(dtype)
+    Y[:, ::97] = 16383
+    Y[:, 50::97] = 16384
+    Y[:5, 100::301] = 2_000_000
+    print(f"[case] large counts {Y.dtype}", flush=True)
+    fit = dv.fit_devil(torch.as_tensor(Y, device="cuda"), X, size_factors=sf, max_iter=3)
+    ref = orc.cpu_fit(Y.astype(np.float64), X, np.log(sf), od_mode=orc.OD_MOM, max_iter=3)
+    close(fit["beta"], ref["beta"], "beta")
+    close(fit["overdispersion"], ref["theta"], "theta")
