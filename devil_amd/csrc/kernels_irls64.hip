@@ -17,7 +17,7 @@ __global__ __launch_bounds__(256) void k_irls_accum(TileDesign td, Counts c,
                                                     const double* __restrict__ beta,
                                                     const double* __restrict__ kvec,
                                                     double* __restrict__ part) {
-  __shared__ double e2[64];
+  __shared__ double e2[kExpTab];
   exp_tab_fill(e2, threadIdx.x, blockDim.x);
   __syncthreads();
   irls_accum_body<P, VC>(td, c, active, nactive, beta, kvec, part, e2, blockIdx.x, gridDim.x);

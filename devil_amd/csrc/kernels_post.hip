@@ -223,7 +223,7 @@ template <int P>
 __global__ __launch_bounds__(256) void k_mom_accum(TileDesign td, ChunkTable ct, Counts c,
                                                    int64_t G, const double* __restrict__ beta,
                                                    double* __restrict__ part) {
-  __shared__ double e2[64];
+  __shared__ double e2[kExpTab];
   exp_tab_fill(e2, threadIdx.x, blockDim.x);
   __syncthreads();
   const int wave = wave_index();
@@ -267,7 +267,7 @@ __global__ __launch_bounds__(256) void k_bread_accum(TileDesign td, ChunkTable c
                                                      int64_t G, const double* __restrict__ beta,
                                                      const double* __restrict__ theta,
                                                      double* __restrict__ part) {
-  __shared__ double e2[64];
+  __shared__ double e2[kExpTab];
   exp_tab_fill(e2, threadIdx.x, blockDim.x);
   __syncthreads();
   const int wave = wave_index();

@@ -1316,7 +1316,7 @@ __device__ __forceinline__ int joint_find(const JointItem* __restrict__ it, int 
 template <int P>
 __global__ __launch_bounds__(256) void k_irls_accum_joint(const JointItem* __restrict__ items,
                                                           int nitems) {
-  __shared__ double e2[64];
+  __shared__ double e2[kExpTab];
   exp_tab_fill(e2, threadIdx.x, blockDim.x);
   __syncthreads();
   const int b = blockIdx.x;

@@ -135,3 +135,28 @@ def test_init_large_counts(dv, orc, dtype):
     ref = orc.cpu_fit(Y.astype(np.float64), X, np.log(sf), od_mode=orc.OD_MOM, max_iter=3)
     close(fit["beta"], ref["beta"], "beta")
     close(fit["overdispersion"], ref["theta"], "theta")
+
+
+@pytest.mark.parametrize("n", [64, 67])
+def test_exponential_table(dv, n):
+    """exp over its range, by the MOM overdispersion of zero counts with an
+    intercept: theta = n / (n - 1) (1 - 1 / mu), mu = exp(beta).  Table entries
+    on both sides of a rounding edge (odd multiples of ln2 / 512) and far ones.
+    Tolerance: sums of n equal terms and exp's two ulps, relative to 1 + 1 / mu."""
+    from devil_amd import _lib as L
+    ln2 = np.log(2.0)
+    x = np.concatenate([ln2 / 512 * np.arange(1, 2048), np.linspace(5, 350, 500),
+                        ln2 / 256 * np.array([255, 256, 257, 511, 512, 100000])])
+    G, lib, ctx = len(x), L.lib(), L.context(0)
+    Y = torch.zeros((G, n), dtype=torch.int32, device="cuda")
+    one, off = (torch.full((n,), v, dtype=torch.float64, device="cuda") for v in (1.0, 0.0))
+    th = torch.empty(G, dtype=torch.float64, device="cuda")
+    b = torch.as_tensor(x, device="cuda")
+    torch.cuda.synchronize()
+    ctx.check(lib.devil_mom_dispersion(ctx.h, Y.data_ptr(), L.COUNTS_I32, G, n, n,
+                                       one.data_ptr(), 1, b.data_ptr(), off.data_ptr(),
+                                       th.data_ptr()))
+    want = n / (n - 1) * -np.expm1(-x)
+    err = np.abs(th.cpu().numpy() - want) / (1 + np.exp(-x))
+    print(f"[case] exp table n={n}: {err.max():.2e}", flush=True)
+    assert err.max() <= (n + 16) * 2.0**-53 * n / (n - 1)
