@@ -13,8 +13,8 @@
 // iteration starts.  A gene that stops makes room for the next one, taken
 // from a counter; nothing returns to the host.
 //
-// FP64 issue bounds it: p + 22 + p (p + 1) / 2 + p instructions per cell and
-// lane (44 for p = 4, as compiled), and for the last genes the latency of one
+// FP64 issue bounds it: p + 21 + p (p + 1) / 2 + p instructions per cell and
+// lane (43 for p = 4, as compiled), and for the last genes the latency of one
 // workgroup's pass.  Against the tile kernel it pads no columns to 16 and no
 // features to 4.  4000 genes x 20000 cells, p = 4 (103347 gene iterations):
 // round kernels 7.9 ms, here 5.6 ms; 1500 x 30001, p = 5: 3.2 and 2.0 ms.  X

@@ -3,15 +3,17 @@
 // One IRLS round (src/beta.cpp:38-46) over the still-active genes is two
 // launches:
 //
-//   k_irls_accum  one wavefront per (16-gene tile, cell chunk).  For every
+//   k_irls_accum  (kernels_irls64.hip, irls_tile.hpp)
+//                 one wavefront per (16-gene tile, cell chunk).  For every
 //                 16-cell block:
 //                   eta' = -X beta      v_mfma_f64_16x16x4f64, D[cell][gene]
 //                   w = exp(eta' - off), r = m w - 1 = (y w - 1) / (1 + k w)
 //                   acc += r' K         v_mfma_f64_16x16x4f64 per 16 columns
 //                 where K holds the distinct columns x_a x_b (a <= b) and x_a
-//                 of the design (the Khatri-Rao product, deduplicated on the
-//                 host).  The tile's 16 x NCP partial sums are written per
-//                 chunk.
+//                 of the design (the Khatri-Rao product, deduplicated at
+//                 set-up); a last tile of one or two columns is summed by
+//                 vector instructions.  The tile's 16 x NCP partial sums
+//                 are written per chunk.
 //   k_irls_update one wavefront per active gene: sums its chunk partials in
 //                 chunk order, forms A = k (X'diag(r)X + X'X) and g = k X'r
 //                 (the column sums of K are precomputed in FP64), solves
