@@ -1111,6 +1111,7 @@ int irls_rounds(devil_ctx* ctx, const TileHost& tl, bool mixed, dv::Counts c, in
   std::vector<GraphRec> grec;       // graph replays: two rounds each
   int k = 0;
   bool graphed = false;
+  DV_HIP(dv::launch_fill_i32(s, nnxt, 1, 0));  // later rounds' by launch_copy_counts
   for (; k < max_iter; ++k) {
     if (k >= 2) {
       DV_HIP(hipEventSynchronize(ctx->round_ev[k & 1]));
@@ -1200,7 +1201,6 @@ int irls_rounds(devil_ctx* ctx, const TileHost& tl, bool mixed, dv::Counts c, in
         DV_HIP(launch_mixed_accum(tl.mixed, s, td, c, p, cur, ncur, bound, beta, kvec, part));
     }
     rec.push_back(ctx->launches.size() > nrec ? (long)nrec : -1);
-    DV_HIP(dv::launch_fill_i32(s, nnxt, 1, 0));
     const int ntile_b = (bound + 15) / 16;
     if (ntile_b <= kSplitTiles && td.nchunk > kSplitSlices) {
       DV_HIP(dv::launch_irls_reduce(s, td.nchunk, td.ncp, kSplitSlices, ntile_b, ncur, part,
@@ -1215,7 +1215,7 @@ int irls_rounds(devil_ctx* ctx, const TileHost& tl, bool mixed, dv::Counts c, in
                                     eps, iters, status, nxt, nnxt, mixed ? kMixedBand : 0.0,
                                     replay, nreplay, bprev));
     }
-    DV_HIP(dv::launch_copy_counts(s, nnxt, 1, ctx->round_counts_dev + (k & 1)));
+    DV_HIP(dv::launch_copy_counts(s, nnxt, 1, ctx->round_counts_dev + (k & 1), ncur));
     DV_HIP(hipEventRecord(ctx->round_ev[k & 1], s));
     std::swap(cur, nxt);
     std::swap(ncur, nnxt);
@@ -1264,6 +1264,7 @@ int driver_rounds(devil_ctx* ctx, const dv::TileDesign& tfull, size_t part_cap, 
   std::vector<int> count{nA};  // count[k]: genes of round k's list
   std::vector<long> rec;       // round k's launch record (-1: none)
   int64_t k = 0;
+  DV_HIP(dv::launch_fill_i32(s, nnxt, 1, 0));  // later rounds' by launch_copy_counts
   for (; k < max_rounds; ++k) {
     if (k >= 2) {
       DV_HIP(hipEventSynchronize(ctx->round_ev[k & 1]));
@@ -1278,9 +1279,8 @@ int driver_rounds(devil_ctx* ctx, const dv::TileDesign& tfull, size_t part_cap, 
       if ((rc = accum(td, bound, k, cur, ncur))) return rc;
     }
     rec.push_back(ctx->launches.size() > nrec ? (long)nrec : -1);
-    DV_HIP(dv::launch_fill_i32(s, nnxt, 1, 0));
     if ((rc = update(td, bound, k, cur, ncur, nxt, nnxt))) return rc;
-    DV_HIP(dv::launch_copy_counts(s, nnxt, 1, ctx->round_counts_dev + (k & 1)));
+    DV_HIP(dv::launch_copy_counts(s, nnxt, 1, ctx->round_counts_dev + (k & 1), ncur));
     DV_HIP(hipEventRecord(ctx->round_ev[k & 1], s));
     std::swap(cur, nxt);
     std::swap(ncur, nnxt);

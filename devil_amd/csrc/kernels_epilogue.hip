@@ -307,14 +307,22 @@ hipError_t launch_padj_finish(hipStream_t s, const double* pval, int64_t G, int 
 
 // dst[i] = src[i], i < n: device counts into pinned host slots (a kernel in
 // the stream rather than a copy-engine transfer, so the next round's kernels
-// need not wait for a copy engine)
-__global__ void k_copy_counts(const int32_t* __restrict__ src, int n, int32_t* __restrict__ dst) {
-  for (int i = threadIdx.x; i < n; i += blockDim.x) dst[i] = src[i];
+// need not wait for a copy engine).  clear (may be null): n counts set to zero
+// in the same launch, those of the list that the round has finished with and
+// the next round appends to; a launch of its own for them took 4.4 us a round.
+__global__ void k_copy_counts(const int32_t* __restrict__ src, int n, int32_t* __restrict__ dst,
+                              int32_t* __restrict__ clear) {
+  for (int i = threadIdx.x; i < n; i += blockDim.x) {
+    dst[i] = src[i];
+    if (clear) clear[i] = 0;
+  }
 }
 
-hipError_t launch_copy_counts(hipStream_t s, const int32_t* src, int n, int32_t* dst) {
+hipError_t launch_copy_counts(hipStream_t s, const int32_t* src, int n, int32_t* dst,
+                              int32_t* clear) {
   if (n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_copy_counts, dim3(1), dim3(n < 256 ? 64 : 256), 0, s, src, n, dst);
+  hipLaunchKernelGGL(k_copy_counts, dim3(1), dim3(n < 256 ? 64 : 256), 0, s, src, n, dst,
+                     clear);
   return hipGetLastError();
 }
 
