@@ -163,9 +163,6 @@ __device__ __forceinline__ T block_sum256(T v, T* sh) {
   return r;
 }
 
-// grid (kStatBlocks, C): per candidate column c and cell range x: the sum of
-// mixed (bits, cell) words (an order-free hash), whether any value is
-// non-zero, and the sum of the values.
 // The c-th candidate column: the design columns, then x_a x_b, a <= b.
 __device__ __forceinline__ ColSpec candidate(int c, int p) {
   if (c < p) return {c, -1};
@@ -178,7 +175,10 @@ __device__ __forceinline__ ColSpec candidate(int c, int p) {
   return {a, a + c};
 }
 
-// part[3][C][kStatBlocks]: hash, non-zero cells, sum (a double's bits)
+// grid (kStatBlocks, C): per candidate column c and cell range x the sum of
+// mixed (bits, cell) words (an order-free hash), whether any value is non-zero
+// and the sum of the values; part[3][C][kStatBlocks] holds the hash, a count of
+// threads with non-zero values and the sum (a double's bits).
 __global__ __launch_bounds__(256) void k_col_stats(const double* __restrict__ X, int64_t n, int p,
                                                    uint64_t* __restrict__ part) {
   __shared__ uint64_t shu[256];
@@ -207,8 +207,9 @@ __global__ __launch_bounds__(256) void k_col_stats(const double* __restrict__ X,
   }
 }
 
-// Sum of m doubles in index order, the rounding errors carried along (Knuth's
-// two-sum), so that the result is as the exact sum rounds.
+// Sum of m doubles in index order; the rounding errors are carried along
+// (Knuth's two-sum) and added at the end.  An infinite sum has no error to add
+// (the two-sum's differences are NaN there).
 __device__ __forceinline__ double sum_carried(const double* v, int64_t stride, int m) {
   double s = 0.0, e = 0.0;
   for (int i = 0; i < m; ++i) {
@@ -217,7 +218,7 @@ __device__ __forceinline__ double sum_carried(const double* v, int64_t stride, i
     e += (s - (t - z)) + (x - z);
     s = t;
   }
-  return s + e;
+  return isfinite(s) ? s + e : s;
 }
 
 // one thread per candidate
