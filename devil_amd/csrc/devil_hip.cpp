@@ -129,20 +129,16 @@ struct DevBuf {
   void* p = nullptr;
   size_t size = 0;
   BlockCache* cache = nullptr;
-  bool borrowed = false;  // the caller's memory
   DevBuf() = default;
   DevBuf(const DevBuf&) = delete;
   DevBuf& operator=(const DevBuf&) = delete;
-  DevBuf(DevBuf&& o) noexcept : p(o.p), size(o.size), cache(o.cache), borrowed(o.borrowed) {
-    o.p = nullptr;
-  }
+  DevBuf(DevBuf&& o) noexcept : p(o.p), size(o.size), cache(o.cache) { o.p = nullptr; }
   DevBuf& operator=(DevBuf&& o) noexcept {
     if (this != &o) {
       release();
       p = o.p;
       size = o.size;
       cache = o.cache;
-      borrowed = o.borrowed;
       o.p = nullptr;
     }
     return *this;
@@ -150,15 +146,9 @@ struct DevBuf {
   ~DevBuf() { release(); }
   void release() {
     if (!p) return;
-    if (borrowed) borrowed = false;
-    else if (cache) cache->give(p, size);
+    if (cache) cache->give(p, size);
     else (void)hipFree(p);
     p = nullptr;
-  }
-  void borrow(void* ptr) {
-    release();
-    p = ptr;
-    borrowed = ptr != nullptr;
   }
   hipError_t alloc(BlockCache* c, size_t bytes) {
     release();
@@ -1901,25 +1891,20 @@ int run_setup(devil_ctx* ctx, const devil_problem* pr, devil_outputs* out, ProbR
     return rc;
   if ((rc = finish_qr(ctx, pr->X, mem, r.d, r.dd))) return rc;
 
-  // per-gene device state (gene-major); what leaves as it is goes straight to
-  // the caller's device memory
-  const bool dev_out = mem == DEVIL_MEM_DEVICE;
+  // per-gene device state (gene-major).  Working memory of the context's own,
+  // also where the outputs are device memory: a call that fails leaves the
+  // caller's outputs untouched, and what it had queued by then writes to no
+  // memory that the caller may free
   DV_ALLOC(r.alpha0, sizeof(double) * G);
   DV_ALLOC(r.kvec, sizeof(double) * G);
   DV_ALLOC(r.beta, sizeof(double) * G * p);
-  if (dev_out) r.theta.borrow(out->theta);
-  else DV_ALLOC(r.theta, sizeof(double) * G);
-  if (dev_out) r.iters.borrow(out->beta_iters);
-  else DV_ALLOC(r.iters, sizeof(int32_t) * G);
-  if (dev_out) r.thit.borrow(out->theta_iters);
-  else DV_ALLOC(r.thit, sizeof(int32_t) * G);
-  if (dev_out && out->status) r.status.borrow(out->status);
-  else DV_ALLOC(r.status, sizeof(int32_t) * G);
-  if (dev_out) r.bread.borrow(out->bread);
-  else DV_ALLOC(r.bread, sizeof(double) * G * p * p);
+  DV_ALLOC(r.theta, sizeof(double) * G);
+  DV_ALLOC(r.iters, sizeof(int32_t) * G);
+  DV_ALLOC(r.thit, sizeof(int32_t) * G);
+  DV_ALLOC(r.status, sizeof(int32_t) * G);
+  DV_ALLOC(r.bread, sizeof(double) * G * p * p);
   r.want_sw = C > 0 && out->sandwich;
-  if (r.want_sw && dev_out) r.sandwich.borrow(out->sandwich);
-  else if (r.want_sw) DV_ALLOC(r.sandwich, sizeof(double) * G * p * p);
+  if (r.want_sw) DV_ALLOC(r.sandwich, sizeof(double) * G * p * p);
 
   hipStream_t s = ctx->stream;
   if (pr->disp_init) {
@@ -2117,8 +2102,16 @@ int run_outputs(devil_ctx* ctx, ProbRun& r) {
   hipStream_t s = ctx->stream;
   const int64_t G = r.G;
   const int p = r.p;
-  if (pr->mem == DEVIL_MEM_DEVICE) {  // the rest is there already
-    DV_HIP(dv::launch_transpose_gp(s, r.beta.as<double>(), G, p, 0, out->beta));
+  if (pr->mem == DEVIL_MEM_DEVICE) {
+    const dv::FitArrays from{r.beta.as<double>(),     r.theta.as<double>(),
+                             r.iters.as<int32_t>(),   r.thit.as<int32_t>(),
+                             r.bread.as<double>(),    r.sandwich.as<double>(),
+                             r.status.as<int32_t>()};
+    const dv::FitArrays to{out->beta,  out->theta,
+                           out->beta_iters, out->theta_iters,
+                           out->bread, r.want_sw ? out->sandwich : nullptr,
+                           out->status};
+    DV_HIP(dv::launch_fit_outputs(s, G, p, from, to));
     DV_HIP(hipStreamSynchronize(s));
     return DEVIL_OK;
   }

@@ -349,6 +349,18 @@ hipError_t launch_bh(hipStream_t s, const double* pval, int64_t G, double* adj, 
 hipError_t launch_transpose_gp(hipStream_t s, const double* src, int64_t G, int p,
                                int to_gene_major, double* dst);
 
+// The results of a fit, copied to the caller's arrays in one launch: beta from
+// gene-major to G x p column-major, the rest as it is (to.sandwich and
+// to.status may be null).
+struct FitArrays {
+  double *beta, *theta;
+  int32_t *iters, *theta_iters;
+  double *bread, *sandwich;
+  int32_t* status;
+};
+hipError_t launch_fit_outputs(hipStream_t s, int64_t G, int p, const FitArrays& from,
+                              const FitArrays& to);
+
 hipError_t launch_fill_i32(hipStream_t s, int32_t* p, int64_t count, int32_t v);
 hipError_t launch_copy_counts(hipStream_t s, const int32_t* src, int n, int32_t* dst,
                               int32_t* clear = nullptr);

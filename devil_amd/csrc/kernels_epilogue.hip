@@ -337,6 +337,23 @@ __global__ void k_transpose_gp(const double* __restrict__ src, int64_t G, int p,
   else dst[g + j * G] = src[g * p + j];
 }
 
+// thread t: element t of the p x p matrices, of beta (column-major) and of the
+// per-gene values: one launch for a transpose and five or six copies
+__global__ void k_fit_outputs(int64_t G, int p, FitArrays from, FitArrays to) {
+  const int64_t total = G * p * p, stride = (int64_t)gridDim.x * blockDim.x;
+  for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < total; t += stride) {
+    to.bread[t] = from.bread[t];
+    if (to.sandwich) to.sandwich[t] = from.sandwich[t];
+    if (t < G * p) to.beta[t] = from.beta[(t % G) * p + t / G];
+    if (t < G) {
+      to.theta[t] = from.theta[t];
+      to.iters[t] = from.iters[t];
+      to.theta_iters[t] = from.theta_iters[t];
+      if (to.status) to.status[t] = from.status[t];
+    }
+  }
+}
+
 __global__ void k_fill_i32(int32_t* p, int64_t count, int32_t v) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < count) p[i] = v;
@@ -378,6 +395,14 @@ hipError_t launch_transpose_gp(hipStream_t s, const double* src, int64_t G, int 
   if (G <= 0) return hipSuccess;
   hipLaunchKernelGGL(k_transpose_gp, dim3((unsigned)((G * p + 255) / 256)), dim3(256), 0, s,
                      src, G, p, to_gene_major, dst);
+  return hipGetLastError();
+}
+
+hipError_t launch_fit_outputs(hipStream_t s, int64_t G, int p, const FitArrays& from,
+                              const FitArrays& to) {
+  if (G <= 0) return hipSuccess;
+  const int64_t blocks = std::min<int64_t>((G * p * p + 255) / 256, 65536);
+  hipLaunchKernelGGL(k_fit_outputs, dim3((unsigned)blocks), dim3(256), 0, s, G, p, from, to);
   return hipGetLastError();
 }
 
