@@ -19,6 +19,7 @@
 #include <vector>
 
 #include "../../include/devil_hip.h"
+#include "column_owners.hpp"
 #include "kernels.hpp"
 #include "newod_driver.hpp"
 #include "port_driver.hpp"
@@ -650,6 +651,7 @@ void shape_design(const ColPlan& cp, int64_t n, int p, int cells_per_block, dv::
   std::memset(&td, 0, sizeof(td));
   for (int a = 0; a < p; ++a) td.kidx_lin[a] = cp.kidx_lin[a];
   for (int q = 0; q < p * (p + 1) / 2; ++q) td.kidx_pair[q] = cp.kidx_pair[q];
+  dv::column_owners(td.kidx_pair, td.kidx_lin, p, td.own_pair, td.own_lin);
   for (size_t c = 0; c < cp.ksum.size() && c < (size_t)DEVIL_NCP_MAX; ++c)
     td.ksum[c] = cp.ksum[c];
   const int ncol = std::max<int>(1, (int)cp.spec.size());

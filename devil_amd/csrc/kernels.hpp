@@ -57,6 +57,8 @@ struct TileDesign {
   const double* eop;     // exp(off) padded with zeros to 16 nblk (FP64 design)
   int kidx_pair[55];     // K column of x_a x_b (packed upper triangle), -1 = zero column
   int kidx_lin[10];      // K column of x_a, -1 = zero column
+  uint64_t own_pair;     // the sums that are the first with their column
+  uint32_t own_lin;      // (column_owners.hpp)
   double ksum[DEVIL_NCP_MAX];  // sum over cells of each K column
 };
 

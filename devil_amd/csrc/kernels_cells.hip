@@ -111,8 +111,10 @@ __device__ __forceinline__ void irls_cells(const TileDesign& td, const CT* __res
 #pragma unroll
   for (int i = 0; i < scatter_left(NV); ++i) {
     const int q = scatter_index<NV>(lane, i);
-    const int col = q < 0 ? -1 : q < NP ? td.kidx_pair[q] : td.kidx_lin[q - NP];
-    if (col >= 0) out[col] = acc[i];
+    if (q < 0) continue;
+    // equal columns share a place: their first sum is the one stored
+    if (q < NP ? (td.own_pair >> q) & 1 : (td.own_lin >> (q - NP)) & 1)
+      out[q < NP ? td.kidx_pair[q] : td.kidx_lin[q - NP]] = acc[i];
   }
 }
 

@@ -1,0 +1,65 @@
+"""Host parts of the library, compiled and run on the CPU."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+CSRC = os.path.join(ROOT, "devil_amd", "csrc")
+
+OWNERS = r"""
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include "column_owners.hpp"
+// every column of a design is written by exactly one sum, the first with it
+int main() {
+  srand(3);
+  for (int t = 0; t < 20000; ++t) {
+    const int p = 1 + t % 10, np = p * (p + 1) / 2, icpt = (t / 10) % 2;
+    int pair[55], lin[10], writes[66], first[66];
+    const int ncol = 1 + rand() % (np + p);
+    for (int a = 0; a < p; ++a) lin[a] = rand() % (ncol + 1) - 1;
+    for (int q = 0; q < np; ++q) pair[q] = rand() % (ncol + 1) - 1;
+    if (icpt) memcpy(pair, lin, sizeof(int) * p);  // x_0 x_b is x_b
+    uint64_t own_pair;
+    uint32_t own_lin;
+    dv::column_owners(pair, lin, p, own_pair, own_lin);
+    memset(writes, 0, sizeof(writes));
+    for (int q = np + p - 1; q >= 0; --q) {
+      const int col = q < np ? pair[q] : lin[q - np];
+      if (col >= 0) first[col] = q;
+    }
+    // a pass with an intercept holds the products alone
+    for (int q = 0; q < (icpt ? np : np + p); ++q) {
+      if (!(q < np ? (own_pair >> q) & 1 : (own_lin >> (q - np)) & 1)) continue;
+      const int col = q < np ? pair[q] : lin[q - np];
+      if (col < 0 || first[col] != q || ++writes[col] != 1) return printf("case %d sum %d\n", t, q);
+    }
+    for (int q = 0; q < np + p; ++q) {
+      const int col = q < np ? pair[q] : lin[q - np];
+      if (col >= 0 && writes[col] != 1) return printf("case %d column %d\n", t, col);
+    }
+  }
+  return 0;
+}
+"""
+
+
+def run(tmp_path, source, compiler, *flags):
+    src = tmp_path / "part.cpp"
+    src.write_text(source)
+    exe = tmp_path / "part"
+    r = subprocess.run([compiler, *flags, "-std=c++17", "-O2", "-I" + CSRC, str(src), "-o",
+                        str(exe)], capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr[-4000:]
+    r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=600)
+    assert r.returncode == 0, r.stdout + r.stderr
+    return r.stdout
+
+
+def test_column_owners(tmp_path):
+    if shutil.which("g++") is None:
+        pytest.skip("no g++")
+    run(tmp_path, OWNERS, "g++")
