@@ -313,21 +313,6 @@ __host__ __device__ inline double lgamma_corr(double x) {
           f * (1.0 / 1188 - f * (691.0 / 360360 - f * (1.0 / 156))))))) / x;
 }
 
-// log B(a, b) with the large-argument forms that avoid cancellation.
-__host__ __device__ inline double lbeta(double a, double b) {
-  const double p = fmin(a, b), q = fmax(a, b);
-  const double half_log_2pi = 0.91893853320467274178;
-  if (p >= 10.0) {
-    const double corr = lgamma_corr(p) + lgamma_corr(q) - lgamma_corr(p + q);
-    return -0.5 * log(q) + half_log_2pi + corr + (p - 0.5) * log(p / (p + q)) +
-           q * log1p(-p / (p + q));
-  } else if (q >= 10.0) {
-    const double corr = lgamma_corr(q) - lgamma_corr(p + q);
-    return lgamma(p) + corr + p - p * log(p + q) + (q - 0.5) * log1p(-p / (p + q));
-  }
-  return lgamma(p) + lgamma(q) - lgamma(p + q);
-}
-
 // 1/d from v_rcp_f64 refined by two Newton steps (about 1 ulp).
 __device__ __forceinline__ double rcp_f64(double d) {
   double r = __builtin_amdgcn_rcp(d);
@@ -372,7 +357,7 @@ __device__ inline double betacf(double a, double b, double x) {
 }
 
 // log of 2*P(T_df > |t|) = log I_{df/(df+t^2)}(df/2, 1/2); exact in log space
-// where the probability underflows.  lb = lbeta(df/2, 1/2), the same for every
+// where the probability underflows.  lb = log B(df/2, 1/2), the same for every
 // gene.
 __device__ inline double log_pt2_upper(double t, double df, double lb) {
   if (isnan(t) || isnan(df) || !(df > 0.0)) return __builtin_nan("");

@@ -375,6 +375,19 @@ hipError_t launch_k_from_alpha(hipStream_t s, const double* alpha0, int64_t G, d
 
 
 
+// log B(a, 1/2) for a >= 1/2, from a = 10 on by the Stirling remainders.
+// lgamma_r: lgamma writes the process's signgam, on which threads with contexts
+// of their own would race.
+static double log_beta_half(double a) {
+  int sign;
+  const double half = lgamma_r(0.5, &sign);
+  if (a >= 10.0) {
+    const double corr = lgamma_corr(a) - lgamma_corr(0.5 + a);
+    return half + corr + 0.5 - 0.5 * log(0.5 + a) + (a - 0.5) * log1p(-0.5 / (0.5 + a));
+  }
+  return half + lgamma_r(a, &sign) - lgamma_r(0.5 + a, &sign);
+}
+
 hipError_t launch_test_de(hipStream_t s, const double* beta, const double* bread,
                           const double* sandwich, int64_t G, int p, double df,
                           const double* contrast, double max_lfc, double* pval,
@@ -382,7 +395,7 @@ hipError_t launch_test_de(hipStream_t s, const double* beta, const double* bread
                           double* adj) {
   if (G <= 0) return hipSuccess;
   const dim3 g1((unsigned)((G + 255) / 256));
-  const double lb = df > 0.0 ? lbeta(0.5 * df, 0.5) : 0.0;
+  const double lb = df > 0.0 ? log_beta_half(0.5 * df) : 0.0;
   hipLaunchKernelGGL(k_test_de, g1, dim3(256), 0, s, beta, bread, sandwich, G, p, df, lb,
                      contrast, max_lfc, pval, logp, lfc);
   hipError_t e = hipGetLastError();

@@ -63,3 +63,19 @@ def test_column_owners(tmp_path):
     if shutil.which("g++") is None:
         pytest.skip("no g++")
     run(tmp_path, OWNERS, "g++")
+
+
+def test_no_call_writes_process_state():
+    """glibc's lgamma stores its sign in the global signgam: two threads with
+    contexts of their own would race on it.  The library calls lgamma_r."""
+    from devil_amd import _lib
+    if shutil.which("nm") is None:
+        pytest.skip("no nm")
+    if not os.path.exists(_lib.LIB_PATH):
+        from devil_amd.build import build
+        build()
+    r = subprocess.run(["nm", "-D", "--undefined-only", _lib.LIB_PATH], capture_output=True,
+                       text=True, check=True)
+    names = {w.split("@")[0] for w in r.stdout.split()}
+    assert "lgamma_r" in names
+    assert not names & {"lgamma", "lgammaf", "lgammal", "gamma", "signgam"}
