@@ -87,7 +87,7 @@ __device__ __forceinline__ void irls_cells(const TileDesign& td, const CT* __res
       if constexpr (ICPT) eta += b[0];
 #pragma unroll
       for (int j = J0; j < P; ++j) eta = fma(b[j], o.x[j], eta);
-      const double w = exp_tab<kExpTabGene>(eta, e2);
+      const double w = exp_tab(eta, e2);
       const double d = fma(k, w, 1.0);
       double r = fma((double)o.y, w, -1.0) * rcp1_f64(d);
       r = in ? r : 0.0;
@@ -124,7 +124,7 @@ __global__ __launch_bounds__(64 * kCellsWaves) void k_irls_cells(
     const int32_t* __restrict__ active, const int32_t* __restrict__ nactive,
     const double* __restrict__ beta, const double* __restrict__ kvec,
     double* __restrict__ part) {
-  __shared__ double e2[kExpTabGene];
+  __shared__ double e2[kExpTab];
   exp_tab_fill(e2, threadIdx.x, blockDim.x);
   __syncthreads();
   const int nA = *nactive;

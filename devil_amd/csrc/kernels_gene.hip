@@ -53,7 +53,7 @@ __host__ __device__ constexpr int gene_slots(int p) { return p <= 5 ? 2 : 1; }
 // LDS of a workgroup.
 template <int NV, int NG, int P>
 struct GeneLds {
-  double e2[kExpTabGene];
+  double e2[kExpTab];
   double part[NG][kGeneMaxWaves * NV];
   double tot[NG][NV + P];  // system entries, then the right-hand side
   double b[NG][P];
@@ -172,7 +172,7 @@ __device__ __forceinline__ void irls_genes(
           if constexpr (ICPT) eta -= b[u][0];
 #pragma unroll
           for (int j = J0; j < P; ++j) eta = fma(-b[u][j], o.x[j], eta);
-          const double w = exp_tab<kExpTabGene>(eta, sh.e2);
+          const double w = exp_tab(eta, sh.e2);
           const double d = fma(k[u], w, 1.0);
           r[u] = fma((double)o.y[u], w, -1.0) * rcp1_f64(d);
           r[u] = in ? r[u] : 0.0;

@@ -79,3 +79,58 @@ def test_no_call_writes_process_state():
     names = {w.split("@")[0] for w in r.stdout.split()}
     assert "lgamma_r" in names
     assert not names & {"lgamma", "lgammaf", "lgammal", "gamma", "signgam"}
+
+
+EXP = r"""
+#include <cmath>
+#include <cstdio>
+#include <random>
+#include <utility>
+#include "device_common.hpp"
+template <size_t J> struct Entry { static constexpr double v = dv::kExp2Tab[J]; };
+template <size_t... J> void fill(double* t, std::index_sequence<J...>) { ((t[J] = Entry<J>::v), ...); }
+int main() {
+  double tab[dv::kExpTab];
+  fill(tab, std::make_index_sequence<dv::kExpTab>());
+  double entry = 0.0;  // largest rounding of an entry, in units of 2^-53
+  for (int j = 0; j < dv::kExpTab; ++j) {
+    const long double t = exp2l((long double)j / dv::kExpTab);
+    entry = fmax(entry, (double)(fabsl(tab[j] - t) / t) * 0x1p53);
+  }
+  std::mt19937_64 g(1);
+  double worst = 0.0;
+  for (int k = 0; k < 6000000; ++k) {
+    const double w = k % 3 == 0 ? 3.0 : k % 3 == 1 ? 30.0 : 700.0;
+    const double x = std::uniform_real_distribution<double>(-w, w)(g);
+    const long double e = expl((long double)x);
+    worst = fmax(worst, (double)(fabsl(dv::exp_tab(x, tab) - e) / e) * 0x1p53);
+  }
+  const double inf = INFINITY;
+  if (dv::exp_tab(800.0, tab) != inf || dv::exp_tab(-800.0, tab) != 0.0 ||
+      !std::isnan(dv::exp_tab(NAN, tab)))
+    return printf("range\n");
+  printf("%.4f %.4f\n", entry, worst);
+  return 0;
+}
+"""
+
+
+def hipcc_host(tmp_path, source):
+    from devil_amd.build import hipcc
+    try:
+        cc = hipcc()
+    except RuntimeError:
+        pytest.skip("no hipcc")
+    return run(tmp_path, source, cc, "-x", "hip", "--offload-host-only")
+
+
+def test_exponential_error(tmp_path):
+    """exp_tab against 64-bit mantissas (expl): its result is t + t (e^r - 1) with
+    a table entry t, so its error is the entry's rounding, the last rounding (at
+    most 1 unit of 2^-53) and the errors of the small term, |e^r - 1| <= 0.0054,
+    which is off by less than three units; the entries are correctly rounded."""
+    entry, worst = map(float, hipcc_host(tmp_path, EXP).split())
+    print(f"exp: table {entry} units of 2^-53, worst {worst}")
+    assert entry <= 1.0
+    assert worst <= entry + 1.0 + 3 * 0.0055
+    assert worst <= 1.75  # what 64 entries reach; with 128 or 256 it is 1.85 or 1.91
