@@ -24,6 +24,7 @@
 #include "../../include/devil_hip.h"
 #include "device_common.hpp"
 #include "kernels.hpp"
+#include "log_fast.hpp"
 #include "tile_common.hpp"
 
 namespace dv {
@@ -420,49 +421,6 @@ __global__ __launch_bounds__(64) void k_bread_finish(TileDesign td, ChunkTable c
 // projection (thin Q of X for the least-squares start, X - mean(X) for the
 // univariate start) and z = log1p(y / s) or log(y + 0.5) - log s.
 // ---------------------------------------------------------------------------
-// log(1 + x) for 0 <= x < 2^52: log_tab's scheme without its special cases, on
-// the bits of u = 1 + x.  Rounding u's mantissa to 7 bits (with the carry into
-// the exponent) gives e and j with m = u 2^-e within 2^-8 of F = 1 + j/128;
-// r = m / F - 1 by one fused multiply-add with the rounded 1/F, whose own
-// error is in the table's logarithm (ln = -log(inv)); x = 0 gives 0 exactly.
-// About 26 instructions against log_tab's 42; the init pass of 4000 genes x
-// 500000 cells, p = 8, takes 3.2 ms against 3.9 (FP64 issue bounds it: this
-// logarithm and 4 matrix instructions of 64 cycles per block of 16 cells).
-struct LogFast {
-  double inv, ln;
-};
-constexpr int kLogFast = 128;
-
-__device__ __forceinline__ void log_fast_fill(LogFast* tab, int tid, int nthreads) {
-  for (int j = tid; j < kLogFast; j += nthreads) {
-    const double f = (double)j * (1.0 / 128), inv = 1.0 / (1.0 + f);
-    tab[j].inv = inv;
-    tab[j].ln = log1p_f64(f) - fma(inv, 1.0 + f, -1.0);
-  }
-}
-
-__device__ __forceinline__ double log1p_fast(double x, const LogFast* tab) {
-  const double u = 1.0 + x;
-  const double c = x - (u - 1.0);  // the rounding error of u
-  const int hi = __double2hiint(u);
-  const int t = hi + 0x1000;
-  const int e20 = (t & 0x7ff00000) - 0x3ff00000;  // 2^20 e
-  const LogFast en = tab[(t >> 13) & (kLogFast - 1)];
-  const double m = __hiloint2double(hi - e20, __double2loint(u));
-  const double scale = __hiloint2double(0x3ff00000 - e20, 0);  // 2^-e
-  const double r = fma(c * scale, en.inv, fma(m, en.inv, -1.0));
-  double q = 1.0 / 7;
-  q = fma(q, r, -1.0 / 6);
-  q = fma(q, r, 1.0 / 5);
-  q = fma(q, r, -1.0 / 4);
-  q = fma(q, r, 1.0 / 3);
-  q = fma(q, r, -0.5);
-  const double lp = fma(r * r, q, r);
-  const double ed = (double)e20;
-  return fma(ed, 6.93147180369123816490e-01 / 1048576, en.ln) +
-         fma(ed, 1.90821492927058770002e-10 / 1048576, lp);
-}
-
 // ZM: 0 no projection (alpha only, rough start), 1 least squares (QR),
 // 2 univariate.
 template <typename CT, int ZM, bool VEC>

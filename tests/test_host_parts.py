@@ -134,3 +134,54 @@ def test_exponential_error(tmp_path):
     assert entry <= 1.0
     assert worst <= entry + 1.0 + 3 * 0.0055
     assert worst <= 1.75  # what 64 entries reach; with 128 or 256 it is 1.85 or 1.91
+
+
+LOG = r"""
+#include <cmath>
+#include <cstdio>
+#include <random>
+#include <utility>
+#include "log_fast.hpp"
+template <size_t J> struct Entry { static constexpr double v = dv::kLogFastLn[J]; };
+template <size_t... J> void fill(dv::LogFast* t, std::index_sequence<J...>) {
+  ((t[J].ln = Entry<J>::v), ...);
+}
+int main() {
+  dv::LogFast tab[dv::kLogFast];
+  fill(tab, std::make_index_sequence<dv::kLogFast>());
+  double entry = 0.0;  // largest rounding of an entry, in halves of its last place
+  for (int j = 0; j < dv::kLogFast; ++j) {
+    tab[j].inv = 1.0 / (1.0 + j / (double)dv::kLogFast);
+    const double ulp = nextafter(tab[j].ln, INFINITY) - tab[j].ln;
+    entry = fmax(entry, (double)fabsl(tab[j].ln + logl(tab[j].inv)) / (0.5 * ulp));
+  }
+  std::mt19937_64 g(1);
+  auto error = [&](double x) {
+    const long double e = log1pl((long double)x);
+    return (double)(fabsl(dv::log1p_fast(x, tab) - e) / e) * 0x1p53;
+  };
+  double wide = 0.0, counts = 0.0;
+  std::uniform_real_distribution<double> lx(-18.0, 34.0), u(0.0, 1.0);
+  std::lognormal_distribution<double> sf(0.0, 0.3);
+  for (int k = 0; k < 3000000; ++k) {
+    wide = fmax(wide, error(exp(lx(g))));
+    counts = fmax(counts, error((1 + (int)(-log(1.0 - u(g)) * 5.0)) / sf(g)));
+  }
+  if (dv::log1p_fast(0.0, tab) != 0.0) return printf("zero\n");
+  printf("%.4f %.4f %.4f\n", entry, wide, counts);
+  return 0;
+}
+"""
+
+
+def test_init_logarithm_error(tmp_path):
+    """log1p_fast against 64-bit mantissas (log1pl).  The worst place is just above
+    x = 1/256, where the result is half of the table entry: the entry's rounding
+    counts 2 units of 2^-53, the last rounding 1, the small term's errors (three
+    roundings of a term below 2^-8, half of the result) well below 1."""
+    entry, wide, counts = map(float, hipcc_host(tmp_path, LOG).split())
+    print(f"log1p: table {entry} half places, worst {wide}, on counts {counts}")
+    assert entry <= 1.01  # correctly rounded (logl's own error aside)
+    assert wide <= 4.0
+    # the general logarithm of the pass (log_tab) reaches 3.17 and 2.23
+    assert wide <= 2.6 and counts <= 2.23
