@@ -678,11 +678,24 @@ struct TileHost {
 };
 
 // The FP64 IRLS takes one workgroup per gene where the design stays in an
-// XCD's L2 (4 MB, shared with the counts of 32 CUs' genes).
+// XCD's L2 (4 MB, shared with the counts of 32 CUs' genes).  Above p = 5 a
+// workgroup holds one gene and reads the design for it alone, twice the bytes
+// of two genes side by side: with many genes in flight the line lies at half.
+// IRLS ms, gene kernel and rounds:
+//   2 MiB  p = 2, 87381 cells:  1100 genes 3.0, 3.7;  5000 genes 8.1, 10.7
+//          p = 5, 43690 cells:  1100 genes 3.0, 3.5;  10000 genes 11.1, 12.5
+//          p = 6, 37449 cells:  300 genes 1.7, 1.9;  1100 2.8, 3.0;  10000 14.5, 13.2
+//          p = 8, 29127 cells:  300 genes 2.2, 2.3;  1100 3.5, 3.9;  2500 5.7, 5.2;
+//                               20000 32.2, 23.0
+//   1 MiB  p = 6, 18724 cells:  2500 genes 2.9, 4.2;  20000 14.1, 14.3
+//          p = 8, 14563 cells:  2500 genes 3.2, 4.1;  20000 14.8, 14.1
+//          p = 10, 11915 cells: 2500 genes 3.4, 5.1;  20000 16.1, 16.2
 constexpr int64_t kGeneDesignBytes = (int64_t)2 << 20;
+constexpr int64_t kGeneFew = 1024;
 
-bool gene_path(const TileHost& tl, int p) {
-  return (int64_t)sizeof(double) * (p + 1) * tl.td.n <= kGeneDesignBytes;
+bool gene_path(const TileHost& tl, int p, int64_t genes) {
+  const bool half = dv::gene_slots(p) == 1 && genes > kGeneFew;
+  return (int64_t)sizeof(double) * (p + 1) * tl.td.n <= kGeneDesignBytes / (half ? 2 : 1);
 }
 
 // Xd, offd, eod: device n x p X, offset and exp(offset).
@@ -1346,7 +1359,7 @@ int run_irls_tiled(devil_ctx* ctx, const TileHost& tl, dv::Counts c, int64_t G, 
     if (max_iter <= 0) DV_HIP(dv::launch_fill_i32(s, status, G, DEVIL_GENE_MAXITER));
     return DEVIL_OK;
   }
-  if (!mixed && gene_path(tl, p))
+  if (!mixed && gene_path(tl, p, G))
     return run_irls_gene(ctx, tl, c, p, nullptr, (int)G, beta, kvec, max_iter, eps, iters,
                          status);
   DevBuf act0, act1, cnt, part, rep, beta0;
@@ -1391,7 +1404,7 @@ int run_irls_tiled(devil_ctx* ctx, const TileHost& tl, dv::Counts c, int64_t G, 
     // FP64 refit of the replay genes from their starting beta
     DV_HIP(dv::launch_restart_genes(s, rep.as<int32_t>(), nr, p, beta0.as<double>(), beta,
                                     iters, status, bprev.as<double>()));
-    if (gene_path(tl, p))
+    if (gene_path(tl, p, nr))
       rc = run_irls_gene(ctx, tl, c, p, rep.as<int32_t>(), nr, beta, kvec, max_iter, eps, iters,
                          status);
     else

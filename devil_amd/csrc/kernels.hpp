@@ -224,6 +224,13 @@ hipError_t launch_polish_select(hipStream_t s, int64_t G, int p, const double* b
                                 int32_t* list, int32_t* nlist);
 hipError_t launch_iota(hipStream_t s, int32_t* p, int n);
 
+// Genes a workgroup of the gene kernel iterates side by side.  Two share each
+// load of X and the offsets and hide each other's latencies; one gene alone
+// needs 8 (p + 1) + 4 bytes a cell from L1, at 64 B per clock and CU about the
+// arithmetic's time.  Above p = 5 the sums of two genes do not fit the
+// registers of two waves a SIMD.
+__host__ __device__ constexpr int gene_slots(int p) { return p <= 5 ? 2 : 1; }
+
 // IRLS of ngenes genes (list[0 .. ngenes), or all when list is null), one
 // workgroup per gene for all its iterations (kernels_gene.hip).  beta holds
 // the starting values; iters and status are written.  max_iter >= 1.  next: a

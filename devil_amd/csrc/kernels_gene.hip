@@ -44,12 +44,6 @@ struct GeneOps {
 
 constexpr int kGeneMaxWaves = 8;
 
-// Genes a workgroup iterates side by side.  Two share each load of X and the
-// offsets and hide each other's latencies; one gene alone needs 8 (p + 1) + 4
-// bytes a cell from L1, at 64 B per clock and CU about the arithmetic's time.
-// Above p = 5 the sums of two genes do not fit the registers of two waves a SIMD.
-__host__ __device__ constexpr int gene_slots(int p) { return p <= 5 ? 2 : 1; }
-
 // LDS of a workgroup.
 template <int NV, int NG, int P>
 struct GeneLds {
