@@ -1003,13 +1003,19 @@ dv::TileDesign round_shape(const dv::TileDesign& td, int nA, int tiles_per_wg,
 }
 
 // An FP64 round of at most kCellsGenes genes runs one gene and chunk per
-// wavefront (launch_irls_cells): enough chunks for kCellsRoundWaves wavefronts
-// (eight a SIMD), of at least kMinCells cells each.  The line: 300 genes x
-// 200001 cells, p = 5, spend 2.66 / 2.17 / 1.91 / 2.10 / 2.26 ms in the
-// accumulates with it at 16 / 48 / 128 / 256 / 512 genes, 4000 x 500000,
-// p = 8, 65.3 / 65.7 / 66.1 / 66.0 / 68.5 ms.
-constexpr int64_t kCellsRoundWaves = 8192;
-constexpr int64_t kMinCells = 256;
+// wavefront (launch_irls_cells): enough chunks for kCellsRoundWaves wavefronts,
+// of at least kMinCells cells each.  The line: 300 genes x 200001 cells, p = 5,
+// spend 2.66 / 2.17 / 1.91 / 2.10 / 2.26 ms in the accumulates with it at 16 /
+// 48 / 128 / 256 / 512 genes, 4000 x 500000, p = 8, 65.3 / 65.7 / 66.1 / 66.0 /
+// 68.5 ms.  kCellsRoundWaves gives lists of up to 64 genes (one column of a tile
+// round's workgroups) kMaxRoundChunks chunks whatever their length, so rounds
+// replayed from a captured graph have the chunks, and the bits, of rounds
+// launched one by one.  IRLS ms with 8192 waves of >= 256 cells, 32768 of >= 256
+// and 32768 of >= 512: 40 genes x 500000 cells, p = 8, 2.31, 2.31, 2.33; 96 x
+// 400000, p = 2, 1.64, 1.64, 1.64; 60 x 140000, p = 10, 2.56, 2.82, 2.58; 64 x
+// 100000, p = 3, 1.18, 1.20, 1.16; 300 x 200001, p = 5, 3.24, 3.28, 3.23.
+constexpr int64_t kCellsRoundWaves = 64 * kMaxRoundChunks;
+constexpr int64_t kMinCells = 512;
 constexpr int kCellsGenes = 96;
 
 dv::TileDesign fp64_shape(const dv::TileDesign& td, int64_t nA, size_t part_cap) {
@@ -1124,8 +1130,9 @@ int irls_rounds(devil_ctx* ctx, const TileHost& tl, bool mixed, dv::Counts c, in
     }
     const int bound = k == 0 ? nA : count[k - 1];
     if (bound <= 0) break;
-    // Once the list fits one workgroup column of tiles, round_shape no longer
-    // depends on its length: the rest of the rounds can replay one graph.
+    // Once the list fits one workgroup column of tiles, a round's shape no
+    // longer depends on its length (round_shape, fp64_shape): the rest of the
+    // rounds can replay one graph.
     const int graph_genes = 16 * tiles_per_wg;
     if (k >= 2 && ctx->tune[DEVIL_TUNE_GRAPH] && bound <= graph_genes && max_iter - k >= 4) {
       // The tail: rounds k, k + 1, ... as replays of two captured rounds

@@ -75,3 +75,32 @@ def test_rule_of_the_gene_kernel(dv, G, n, p, one_launch):
     finally:
         ctx.set_timing(False)
     assert (launches == 1) == one_launch, launches
+
+
+def test_graph_tail_of_the_round_kernels(dv, orc):
+    """The FP64 rounds of a row too long for the gene kernel, replayed from a
+    captured graph (DEVIL_TUNE_GRAPH) and launched one by one: the lists of up to
+    64 genes have the same chunks whatever their length, so the results have the
+    same bits.  The graph records two rounds a launch: fewer timed launches."""
+    from devil_amd import _lib as L
+    r = np.random.default_rng(13)
+    n, p, G = 120000, 8, 40
+    X = np.column_stack([np.ones(n), r.uniform(size=n) < 0.4] +
+                        [r.normal(size=n) for _ in range(p - 2)]).astype(np.float64)
+    Y, sf = counts(r, X, G)
+    Y[0] = 0  # more iterations than the others
+    Y[0, ::9000] = 1
+    Yd = torch.as_tensor(Y, device="cuda")
+    ctx = dv.context(0)
+    beta, launches = {}, {}
+    try:
+        ctx.set_timing(True)
+        for graph in (1, 0):
+            ctx.set_tuning(L.TUNE_GRAPH, graph)
+            beta[graph] = check(dv, orc, Y, X, sf, Yd)
+            launches[graph] = ctx.kernel_stats()["irls_fp64"][0]
+    finally:
+        ctx.set_tuning(L.TUNE_GRAPH, 0)
+        ctx.set_timing(False)
+    assert launches[1] < launches[0], launches
+    np.testing.assert_array_equal(beta[1], beta[0])
