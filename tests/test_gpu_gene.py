@@ -116,3 +116,78 @@ def test_design_setup(dv, orc):
     ref = orc.cpu_fit(Y.astype(np.float64), Xc, np.log(sf), od_mode=orc.OD_NONE)
     # the condition number 2e3 enters the normal equations squared: 4e6 * 2^-53
     np.testing.assert_allclose(fit["beta"].cpu().numpy(), ref["beta"], rtol=1e-8, atol=1e-8)
+
+
+# A workgroup holds two genes (p <= 5) only where the genes outnumber the
+# workgroups: 1024 up to 16384 cells, 512 above.  Few cells keep the oracle
+# quick; a workgroup's step is 256 (512) cells.
+@pytest.mark.parametrize("intercept", [True, False])
+@pytest.mark.parametrize("p", [1, 2, 3, 4, 5])
+def test_two_genes_side_by_side(dv, orc, p, intercept):
+    """Three full steps (the pipeline's two buffers end on the odd one) and a
+    partial one."""
+    check(dv, orc, *problem(1400, 3 * 256 + 37, p, intercept))
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("n", [200, 256, 512, 4 * 256 + 1])
+def test_two_genes_steps_and_count_types(dv, orc, n, dtype):
+    """No full step, whole steps only, an even number of steps and a remainder."""
+    check(dv, orc, *problem(1100, n, 3, dtype=dtype))
+
+
+@pytest.mark.parametrize("n,p,intercept", [(16385, 2, True), (16896, 5, False)])
+def test_two_genes_in_wide_workgroups(dv, orc, n, p, intercept):
+    """512 threads: more than 512 genes, 32 full steps and a remainder, and 33."""
+    check(dv, orc, *problem(600, n, p, intercept))
+
+
+@pytest.mark.parametrize("p", [2, 4])
+def test_pairing_does_not_change_bits(dv, p):
+    """Which genes share a workgroup depends on timing; a gene's result does not:
+    two fits have the same bits, and a gene fitted in a launch of its own (one
+    gene per workgroup) has them too."""
+    Y, X, sf = problem(1500, 900, p, seed=3)
+    Yd = torch.as_tensor(Y, device="cuda")
+    fit = lambda y: dv.fit_devil(y, X, size_factors=sf, overdispersion=False,
+                                 init_overdispersion=0.7, init_mode="rough")
+    print(f"[case] pairing p={p}", flush=True)
+    a, b, few = fit(Yd), fit(Yd), fit(Yd[:40])
+    for x, y in ((a, b), (a, few)):
+        m = y["beta"].shape[0]
+        np.testing.assert_array_equal(x["beta"][:m].cpu().numpy(), y["beta"].cpu().numpy())
+        np.testing.assert_array_equal(x["iterations"]["beta_iters"][:m].cpu().numpy(),
+                                      y["iterations"]["beta_iters"].cpu().numpy())
+
+
+@pytest.mark.parametrize("sign", [1, -1])
+def test_one_step_from_zero_counts(dv, sign):
+    """One iteration on zero counts with an intercept is a closed expression of w
+    = exp(-beta - off): r = -1 / (1 + k w), A = k (sum r + n), step = sum r / (sum
+    r + n) = -1 / (k w) whatever n is.  Offsets over both signs; bar: sum r is
+    within n 2^-53 and the reciprocal within 2.2e-15, and sum r + n = n k w / (1 +
+    k w) divides both by the cancellation k w / (1 + k w)."""
+    from devil_amd import _lib as L
+    n, k = 128, 2.0
+    b = sign * np.linspace(0.0, 3.0, 700)
+    G = len(b)
+    Y = torch.zeros((G, n), dtype=torch.int32, device="cuda")
+    one, off = (torch.full((n,), v, dtype=torch.float64, device="cuda") for v in (1.0, 0.0))
+    beta = torch.as_tensor(b, device="cuda").clone()
+    alpha = torch.full((G,), 1.0 / k, dtype=torch.float64, device="cuda")
+    it, st = (torch.empty(G, dtype=torch.int32, device="cuda") for _ in range(2))
+    ctx = dv.context(0)
+    torch.cuda.synchronize()
+    ctx.check(dv.lib().devil_beta_fit(ctx.h, Y.data_ptr(), L.COUNTS_I32, G, n, n,
+                                      one.data_ptr(), 1, beta.data_ptr(), off.data_ptr(),
+                                      alpha.data_ptr(), 1, 1e-3, L.PREC_FP64, it.data_ptr(),
+                                      st.data_ptr()))
+    step = beta.cpu().numpy() - b
+    kw = k * np.exp(-b)
+    err = np.abs(step * kw + 1.0)
+    # w's error (2 units of 2^-53), the reciprocal's, sum r's and the division's,
+    # over the cancellation; the rounding of beta + step against the step
+    bar = (2.2e-15 + 12 * 2.0**-53) * (1 + kw) / kw + 4 * 2.0**-53 * (1 + np.abs(b) * kw)
+    print(f"[case] one step from zero counts, sign {sign}: {(err / bar).max():.2f} of the bar",
+          flush=True)
+    assert np.all(err <= bar), (err / bar).max()

@@ -104,3 +104,69 @@ def test_graph_tail_of_the_round_kernels(dv, orc):
         ctx.set_timing(False)
     assert launches[1] < launches[0], launches
     np.testing.assert_array_equal(beta[1], beta[0])
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("G", [40, 96, 97, 130])
+def test_count_types_of_the_round_kernels(dv, orc, G, dtype):
+    """float32 and float64 counts, rows of odd length in an array of longer rows
+    (leading dimension n + 6, a view that starts at an odd element): one gene
+    per wavefront up to 96 genes, tiles above."""
+    r = np.random.default_rng(G)
+    n = 52428 + 3
+    X = np.column_stack([np.ones(n), r.uniform(size=n) < 0.5] +
+                        [r.normal(size=n) for _ in range(2)]).astype(np.float64)
+    Y, sf = counts(r, X, G, dtype)
+    wide = torch.full((G, n + 6), -1.0, dtype=torch.as_tensor(Y).dtype, device="cuda")
+    wide[:, 3:n + 3] = torch.as_tensor(Y, device="cuda")
+    check(dv, orc, Y, X, sf, wide[:, 3:n + 3])
+
+
+def distinct_columns(X):
+    """Distinct non-zero columns among the design's and their products."""
+    p = X.shape[1]
+    cols = [X[:, a] for a in range(p)] + [X[:, a] * X[:, b] for a in range(p)
+                                          for b in range(a, p)]
+    return len({c.tobytes() for c in np.array(cols) + 0.0 if c.any()})
+
+
+@pytest.mark.parametrize("columns", [2, 17, 18, 19])
+@pytest.mark.parametrize("patients", [0, 3])
+def test_last_column_tile_of_long_rows(dv, orc, columns, patients):
+    """Tiles of long rows (more than 96 genes) whose last column tile holds two
+    columns and is the only one (an intercept and a 0/1 condition), one, two
+    (both summed by vector instructions) and three (a matrix tile)."""
+    r = np.random.default_rng(columns)
+    n = 87381 + 5 if columns == 2 else 40000
+    b = (r.uniform(size=n) < 0.4).astype(float)
+    lv = r.integers(0, 3, n)
+    z = r.normal(size=(n, 4))
+    X = np.column_stack({
+        2: [np.ones(n), b],
+        17: [z[:, 0], z[:, 1], z[:, 2], b, 1 - b],          # no column of ones
+        18: [np.ones(n), lv == 1, lv == 2, z[:, 0], z[:, 1], z[:, 2]],
+        19: [z[:, 0], z[:, 1], z[:, 2], b, 0.5 * (lv == 1)],
+    }[columns]).astype(np.float64)
+    assert distinct_columns(X) == columns
+    p = X.shape[1]
+    if 8 * (p + 1) * n <= 2 << 20:
+        n = (2 << 20) // (8 * (p + 1)) + 9
+        X = np.resize(X, (n, p))
+        assert distinct_columns(X) == columns
+    G = 130
+    Y, sf = counts(r, X, G)
+    lab = np.sort(r.integers(0, patients, n)) if patients else None
+    ends = None if lab is None else np.cumsum(np.bincount(lab)).astype(np.int32)
+    print(f"[case] columns={columns} p={p} n={n} patients={patients}", flush=True)
+    fit = dv.fit_devil(torch.as_tensor(Y, device="cuda"), X, size_factors=sf, clusters=lab)
+    ref = orc.cpu_fit(Y.astype(np.float64), X, np.log(sf), od_mode=orc.OD_MOM,
+                      clusters_ends=ends, n_threads=8)
+    np.testing.assert_array_equal(fit["iterations"]["beta_iters"].cpu(), ref["beta_iters"])
+    for key, want in (("beta", "beta"), ("overdispersion", "theta"),
+                      ("beta_sandwiches_null", "bread"), ("beta_sandwiches", "sandwich")):
+        if fit[key] is None:
+            continue
+        x, y = fit[key].cpu().numpy().reshape(G, -1), np.asarray(ref[want]).reshape(G, -1)
+        scale = np.maximum(np.abs(y).max(axis=1, keepdims=True), 1e-12)
+        err = np.abs(x - y) / scale
+        assert np.all(np.isfinite(err)) and err.max() <= 1e-8, (key, err.max())
