@@ -827,11 +827,17 @@ int tile_from_device(devil_ctx* ctx, const double* X, const double* offset, int6
 // max(2048, n / 64) cells, never straddling a patient block; the count is
 // rounded up to a multiple of 8 with empty chunks (one XCD per chunk).  With
 // few genes the ranges are shorter, so that the passes' waves (a 16-gene tile
-// and a range each) fill the GPU: kPostWaves of them, down to 128 cells and
-// up to 256 ranges.  64 genes x 2000 cells ran on 4 waves of 125 blocks each,
-// 97 us for the init pass and 109 us for the bread; 64 waves take 11 and
-// 10 us.  genes = 0 keeps the long ranges: the mixed clustered pass sums the
-// pair columns in FP32 over a range, so its ranges set its rounding.
+// and a range each) fill the GPU: kPostWaves of them, of at least 128 cells and
+// n / 256 (some more than 256 ranges, and one more per patient).  64 genes x
+// 2000 cells ran on 4 waves of 125 blocks each, 97 us for the init pass and 109
+// us for the bread; 64 waves take 11 and 10 us.  Init and bread stages, us, at
+// 1024 / 4096 / 16384 waves: 300 genes x 200000 cells, p = 6, 211 / 239 / 261
+// and 281 / 250 / 262, 1500 x 30001, p = 6, 132 / 128 / 211 and 196 / 171 /
+// 197, 300 x 20000, p = 2, 56 / 99 / 99 and 40 / 58 / 58 (the finish sums the
+// ranges); with at least 64 / 128 / 256 cells: 64 x 2000, p = 2, 22 / 19 / 24 and
+// 16 / 15 / 17, 64 x 20000, p = 2, 114 / 71 / 48 and 73 / 49 / 34.  genes = 0
+// keeps the long ranges: the mixed clustered pass sums the pair columns in FP32
+// over a range, so its ranges set its rounding.
 constexpr int64_t kPostWaves = 4096;
 
 struct ChunkHost {

@@ -8,7 +8,7 @@
 // the caller's layout, the sums of a chunk stay in registers and end in one
 // reduce-scatter.  The four wavefronts of a workgroup take four genes over the
 // same cells (X once from L2), and chunks are dealt to the XCDs as in the tile
-// kernel (X once from HBM).  Issue-bound at p + 22 + p (p + 1) / 2 + p vector
+// kernel (X once from HBM).  Issue-bound at p + 23 + p (p + 1) / 2 + p vector
 // instructions per cell and lane where the rows fill the GPU, latency-bound
 // below.  40 genes x 500000 cells, p = 8: 39 rounds, 6.9 ms in the tile
 // kernel, 1.4 ms here.

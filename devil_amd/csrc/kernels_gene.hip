@@ -4,7 +4,7 @@
 // The round kernels (kernels_tile.hip) take four launches per iteration of
 // the whole problem.  Where a round's work is microseconds the launches are
 // the time: 2000 genes x 5000 cells, p = 2, ran 123 rounds of 36 us (4.4 ms)
-// for 85 us of arithmetic, and runs 0.52 ms here; 64 genes x 2000 cells 71
+// for 85 us of arithmetic, and runs 0.55 ms here; 64 genes x 2000 cells 71
 // rounds, 3.2 ms, and 0.16 ms here.  A workgroup keeps a gene until it stops:
 // its threads stride over the cells (lane = cell, so counts and the columns
 // of X are read coalesced, in the caller's layout), each lane sums r x_a x_b
@@ -13,14 +13,21 @@
 // iteration starts.  A gene that stops makes room for the next one, taken
 // from a counter; nothing returns to the host.
 //
-// FP64 issue bounds it: p + 21 + p (p + 1) / 2 + p instructions per cell and
-// lane (43 for p = 4, as compiled), and for the last genes the latency of one
-// workgroup's pass.  Against the tile kernel it pads no columns to 16 and no
-// features to 4.  4000 genes x 20000 cells, p = 4 (103347 gene iterations):
-// round kernels 7.9 ms, here 5.6 ms; 1500 x 30001, p = 5: 3.2 and 2.0 ms.  X
-// and the offsets are read once per iteration of two genes, from the XCD's
-// L2, which is why the caller takes this path only where they fit there
-// (launch_irls_gene's callers hold the rule).
+// While all workgroups have genes, FP64 issue bounds it: 48 vector instructions
+// per cell and lane for p = 4 (SQ_INSTS_VALU), about p + 22 + p (p + 1) / 2 + p
+// and the loop around them; at the end the iterations of the genes that stop
+// last, one workgroup's pass each.  4000 genes x 20000 cells, p = 4 (103347 gene
+// iterations, the longest 148): 2.5 ms of vector issue at 2.4 GHz (3.4 at the
+// rate a loop of FP64 multiply-adds reaches) in a 5.4 ms kernel.  The longest
+// gene alone takes 1.94 ms (13.1 us an iteration), the 100 genes with more than
+// 74 iterations 1.96, the other 3900 3.4; handed out longest first all take
+// 3.7, so the rest is long genes that started late.  2000 x 5000, p = 2: 0.55
+// ms, the longest gene alone 0.47 (123 iterations of 3.8 us).  Against the tile
+// kernel it pads no columns to 16 and no features to 4: 4000 x 20000, p = 4,
+// round kernels 7.9 ms, here 5.4; 1500 x 30001, p = 5: 3.2 and 1.9 ms.  X and
+// the offsets are read once per iteration of two genes (one above p = 5), from
+// the XCD's L2, which is why the caller takes this path only where they fit
+// there (launch_irls_gene's callers hold the rule).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -326,7 +333,14 @@ hipError_t launch_gene_p(hipStream_t s, const GeneDesign& gd, Counts c, const in
                          int max_iter, double eps, int32_t* iters, int32_t* status) {
   // Four wavefronts fill a CU's SIMDs once and leave room for other genes'
   // workgroups beside them (their solves overlap this one's cells); long rows
-  // take eight, which shortens the last genes' iterations.
+  // take eight, which shortens the last genes' iterations.  IRLS ms with 256
+  // and 512 threads:
+  //   10000 genes x 4000 cells     p = 2 0.93, 0.88;  p = 5 1.62, 2.15;  p = 8 2.88, 4.90
+  //   3000 x 16384                 p = 2 1.45, 1.17;  p = 5 2.06, 1.80;  p = 8 3.60, 4.05
+  //   10000 x 16384                p = 2 2.84, 2.48;  p = 5 4.54, 4.57;  p = 8 9.52, 10.6
+  //   3000 x 30000                 p = 2 2.24, 1.80;  p = 5 3.64, 3.13
+  // (p = 2 would take 512 from 4000 cells on, p = 8 256 throughout; the line is
+  // p = 5's.)
   const int T = gd.n <= 16384 ? 256 : 512;
   const int grid = std::min(ngenes, T == 256 ? 1024 : 512);
   const hipError_t e = launch_fill_i32(s, next, 1, grid);

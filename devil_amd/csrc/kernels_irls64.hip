@@ -1,6 +1,6 @@
 // gfx950 FP64 IRLS accumulate of one round, 16-gene tiles (irls_tile.hpp; the
 // scheme is described in kernels_tile.hip).  FP64 issue bounds it: per block
-// of 16 cells ~137 vector instructions and, at 64 cycles each on the same
+// of 16 cells ~145 vector instructions and, at 64 cycles each on the same
 // units, ceil(p / 4) + 4 per 16-column tile matrix instructions, which is why
 // a last tile of one or two columns is summed by vector instructions
 // (vcols_of).

@@ -21,9 +21,11 @@
 //                 reference stopping rules; unconverged genes are appended to
 //                 the next active list.
 //
-// Chunking is fixed per fit and a gene's row of an MFMA product depends only
-// on that gene's operand row, so results do not depend on the active-list
-// order or on how many genes share a tile.
+// A gene's row of an MFMA product depends only on that gene's operand row, so
+// results do not depend on the active list's order or on a gene's place in it.
+// A round's chunks (and, for few genes, its kernel) follow from the number of
+// active genes, so which genes share a fit can move the last bits of a gene's
+// FP64 sums; the same fit always has the same bits.
 //
 // v_mfma_f64_16x16x4f64 lane layout (checked on gfx950): lane l supplies
 // A[l % 16][l / 16] and B[l / 16][l % 16]; register r of the result holds
@@ -1153,7 +1155,8 @@ __global__ void k_merge_flags(int32_t* __restrict__ status, const int32_t* __res
 // One workgroup per active gene.  Its threads sum the chunk partials in
 // kUpdSlices interleaved slices per column (two accumulators each, so a
 // round of up to 512 chunks keeps many loads in flight), the slices are
-// added in LDS, and one lane runs the p x p solve.
+// added in LDS, and the first wavefront runs the p x p solve (one lane up to
+// p = 2, above a row per lane).
 constexpr int kUpdThreads = 256;
 constexpr int kUpdSlices = 16;
 

@@ -6,9 +6,9 @@
 namespace dv {
 
 // Lane sums of V values: after scatter_step<V, 32> a lane's v[i] holds the
-// wave's sum of value scatter_index<V>(lane, i), i < scatter_left(V).  Each step halves the values a lane holds and pairs
-// lanes 32, 16, 8, 4, 2, 1 apart, so the 64-lane sums of V values take about
-// V exchanges instead of 6 V.
+// wave's sum of value scatter_index<V>(lane, i), i < scatter_left(V).  Each
+// step halves the values a lane holds and pairs lanes 32, 16, 8, 4, 2, 1 apart,
+// so the 64-lane sums of V values take about V exchanges instead of 6 V.
 __host__ __device__ constexpr int scatter_left(int V) {
   for (int i = 0; i < 6; ++i) V = (V + 1) / 2;
   return V;
