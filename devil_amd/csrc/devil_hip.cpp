@@ -690,10 +690,19 @@ struct TileHost {
 //   1 MiB  p = 6, 18724 cells:  2500 genes 2.9, 4.2;  20000 14.1, 14.3
 //          p = 8, 14563 cells:  2500 genes 3.2, 4.1;  20000 14.8, 14.1
 //          p = 10, 11915 cells: 2500 genes 3.4, 5.1;  20000 16.1, 16.2
+// From p = 9 on the kernel's registers leave two wavefronts a SIMD and nothing
+// beside a gene's solve; the rounds solve all genes' systems side by side, and
+// have the better of it with tens of thousands of genes:
+//   100 cells   p = 8: 60000 genes 11.3, 18.0; 150000 26.5, 37.0
+//               p = 9: 20000 8.1, 11.0; 60000 21.9, 21.6; 150000 52.9, 45.3
+//               p = 10: 20000 9.0, 11.2; 60000 23.6, 20.9; 150000 56.5, 42.8
+//   1000 cells  p = 10: 20000 6.4, 9.6; 60000 16.7, 16.8; 150000 39.5, 32.5
+//   8000 cells  p = 10: 20000 12.2, 13.9; 60000 35.0, 31.1
 constexpr int64_t kGeneDesignBytes = (int64_t)2 << 20;
-constexpr int64_t kGeneFew = 1024;
+constexpr int64_t kGeneFew = 1024, kGeneMany = 40000;
 
 bool gene_path(const TileHost& tl, int p, int64_t genes) {
+  if (p > 8 && genes > kGeneMany) return false;
   const bool half = dv::gene_slots(p) == 1 && genes > kGeneFew;
   return (int64_t)sizeof(double) * (p + 1) * tl.td.n <= kGeneDesignBytes / (half ? 2 : 1);
 }

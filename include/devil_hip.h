@@ -292,7 +292,9 @@ enum { DEVIL_TUNE_MIXED_KERNEL = 0,  /* DEVIL_MIXED_* (default AUTO) */
                                         as replays of a captured two-round hipGraph
                                         (accumulate, clear, update, count copy, twice);
                                         0 (default): launched one by one, queued ahead of the
-                                        count reads (the same speed; per-kernel timing) */
+                                        count reads (the same speed; per-kernel timing);
+                                        FP64 fits of short rows run every iteration in one
+                                        launch and have no rounds */
        DEVIL_TUNE_BATCH_GENES = 7,   /* host-resident counts are uploaded and fitted in gene
                                         batches sized by free device memory (up to 8 GiB);
                                         N > 0 caps a batch at N genes, 0 (default): no cap */
@@ -330,7 +332,8 @@ enum { DEVIL_KERNEL_IRLS_FP64 = 0, DEVIL_KERNEL_IRLS_MIXED = 1,
        DEVIL_N_KERNELS = 3 };
 /* launches: number of launches; ms: summed device milliseconds (HIP events
  * on the context's stream around each launch); bytes: summed algorithmic
- * bytes (count element size x n x active genes of each launch). */
+ * bytes (count element size x n x active genes of each launch; the one launch
+ * of a short-row FP64 fit counts every gene's iterations). */
 int devil_kernel_stats(const devil_ctx *ctx, int32_t kernel, int64_t *launches, double *ms,
                        double *bytes);
 

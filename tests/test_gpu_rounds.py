@@ -57,11 +57,12 @@ def test_equal_columns_of_different_products(dv, orc, intercept):
 
 @pytest.mark.parametrize("G,n,p,one_launch", [
     (1100, 43690, 5, True), (1024, 37449, 6, True), (1025, 18724, 6, True),
-    (1025, 18725, 6, False), (1025, 37449, 6, False), (1025, 11916, 10, False)])
+    (1025, 18725, 6, False), (1025, 37449, 6, False), (1025, 11916, 10, False),
+    (40001, 64, 8, True), (40000, 64, 9, True), (40001, 64, 9, False)])
 def test_rule_of_the_gene_kernel(dv, G, n, p, one_launch):
     """The gene kernel (one launch for the whole IRLS) up to 2 MiB of design, and
-    above five columns with more than 1024 genes up to 1 MiB: with one gene per
-    workgroup the rounds are faster beyond."""
+    above five columns with more than 1024 genes up to 1 MiB, above eight up to
+    40000 genes: with one gene per workgroup the rounds are faster beyond."""
     print(f"[case] rule G={G} n={n} p={p}", flush=True)
     gen = torch.Generator(device="cuda").manual_seed(n)
     Y = torch.poisson(torch.full((G, n), 2.0, device="cuda"), generator=gen).to(torch.int32)
