@@ -677,34 +677,37 @@ struct TileHost {
   DevBuf Xp, offp, eop, Kp, Xf, offf, Kf, xab, offl, kg, kh, kh2;
 };
 
-// The FP64 IRLS takes one workgroup per gene where the design stays in an
-// XCD's L2 (4 MB, shared with the counts of 32 CUs' genes).  Above p = 5 a
-// workgroup holds one gene and reads the design for it alone, twice the bytes
-// of two genes side by side: with many genes in flight the line lies at half.
-// IRLS ms, gene kernel and rounds:
-//   2 MiB  p = 2, 87381 cells:  1100 genes 3.0, 3.7;  5000 genes 8.1, 10.7
-//          p = 5, 43690 cells:  1100 genes 3.0, 3.5;  10000 genes 11.1, 12.5
-//          p = 6, 37449 cells:  300 genes 1.7, 1.9;  1100 2.8, 3.0;  10000 14.5, 13.2
-//          p = 8, 29127 cells:  300 genes 2.2, 2.3;  1100 3.5, 3.9;  2500 5.7, 5.2;
-//                               20000 32.2, 23.0
-//   1 MiB  p = 6, 18724 cells:  2500 genes 2.9, 4.2;  20000 14.1, 14.3
-//          p = 8, 14563 cells:  2500 genes 3.2, 4.1;  20000 14.8, 14.1
-//          p = 10, 11915 cells: 2500 genes 3.4, 5.1;  20000 16.1, 16.2
-// From p = 9 on the kernel's registers leave two wavefronts a SIMD and nothing
-// beside a gene's solve; the rounds solve all genes' systems side by side, and
-// have the better of it with tens of thousands of genes:
-//   100 cells   p = 8: 60000 genes 11.3, 18.0; 150000 26.5, 37.0
-//               p = 9: 20000 8.1, 11.0; 60000 21.9, 21.6; 150000 52.9, 45.3
-//               p = 10: 20000 9.0, 11.2; 60000 23.6, 20.9; 150000 56.5, 42.8
-//   1000 cells  p = 10: 20000 6.4, 9.6; 60000 16.7, 16.8; 150000 39.5, 32.5
-//   8000 cells  p = 10: 20000 12.2, 13.9; 60000 35.0, 31.1
-constexpr int64_t kGeneDesignBytes = (int64_t)2 << 20;
-constexpr int64_t kGeneFew = 1024, kGeneMany = 40000;
+// The FP64 IRLS takes one workgroup per gene (launch_irls_gene) where the design
+// stays in an XCD's L2 (4 MB, shared with the counts of 32 CUs' genes) and the
+// rounds are not faster.  What the gene kernel saves are the rounds of the last
+// genes; what it costs is the design read once per iteration of two genes,
+// above p = 5 of one, and from p = 9 on (8 without an intercept) registers that
+// leave two wavefronts a SIMD and nothing beside a gene's solve; without an
+// intercept p more sums per cell.  So the line sinks with the number of genes.
+// IRLS time of the rounds over the gene kernel's, designs of normal columns with
+// an intercept / without / one-hot:
+//   genes                1500            4000            10000           20000
+//   p = 5, 20000 cells   1.6 / 1.2 / 1.6 1.4 / 1.1 / 1.3 1.2 / 1.0 / 1.2 1.1 / 1.0 / 1.2
+//   p = 7, 6000 cells    2.2 / 1.5 / 2.1 2.1 / 1.6 / 2.1 1.6 / 1.3 / 1.6 1.3 / 1.1 / 1.3
+//   p = 7, 13000 cells   1.5 / 1.2 / 1.5 1.3 / 1.2 / 1.2 1.0 / .94 / 1.1 .97 / .91 / .95
+//   p = 8, 2000 cells    2.9 / 1.5 / 3.1 3.2 / 1.9 / 3.1 2.2 / 1.1 / 2.1 1.7 / .92 / 1.7
+//   p = 8, 11000 cells   1.6 / .98 / 1.4 1.4 / 1.0 / 1.3 1.1 / .84 / 1.1 1.0 / .81 / .94
+//   p = 10, 2000 cells   2.0 / 1.4 / 1.9 2.2 / 1.6 / 1.9 1.3 / .88 / 1.3 1.2 / .77 / 1.1
+//   p = 10, 11000 cells  1.4 / .87 / 1.2 1.2 / .94 / .98 1.1 / .77 / .89 .92 / .74 / .76
+// and, where some genes take many iterations, 8 (p + 1) n = 2 MiB: p = 6 1.10 with
+// 300 genes, 1.07 with 1100, .91 with 10000, p = 8 1.07, 1.11, .77; p = 10, 100
+// cells: 1.25 with 20000 genes, .88 with 60000.
+int64_t gene_design_bytes(int p, int intercept, int64_t genes) {
+  constexpr int64_t KiB = 1024;
+  if (genes <= 1024) return 2048 * KiB;
+  if (dv::gene_slots(p) == 2) return (intercept ? 2048 : 1024) * KiB;
+  if (genes <= 5000) return (intercept ? 1024 : 704) * KiB;
+  if (p + !intercept <= 8) return 512 * KiB;
+  return intercept && genes <= 20000 ? 256 * KiB : 0;
+}
 
 bool gene_path(const TileHost& tl, int p, int64_t genes) {
-  if (p > 8 && genes > kGeneMany) return false;
-  const bool half = dv::gene_slots(p) == 1 && genes > kGeneFew;
-  return (int64_t)sizeof(double) * (p + 1) * tl.td.n <= kGeneDesignBytes / (half ? 2 : 1);
+  return (int64_t)sizeof(double) * (p + 1) * tl.td.n <= gene_design_bytes(p, tl.intercept, genes);
 }
 
 // Xd, offd, eod: device n x p X, offset and exp(offset).

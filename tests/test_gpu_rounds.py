@@ -55,23 +55,25 @@ def test_equal_columns_of_different_products(dv, orc, intercept):
     np.testing.assert_array_equal(a, b)
 
 
-@pytest.mark.parametrize("G,n,p,one_launch", [
-    (1100, 43690, 5, True), (1024, 37449, 6, True), (1025, 18724, 6, True),
-    (1025, 18725, 6, False), (1025, 37449, 6, False), (1025, 11916, 10, False),
-    (40001, 64, 8, True), (40000, 64, 9, True), (40001, 64, 9, False)])
-def test_rule_of_the_gene_kernel(dv, G, n, p, one_launch):
-    """The gene kernel (one launch for the whole IRLS) up to 2 MiB of design, and
-    above five columns with more than 1024 genes up to 1 MiB, above eight up to
-    40000 genes: with one gene per workgroup the rounds are faster beyond."""
-    print(f"[case] rule G={G} n={n} p={p}", flush=True)
+@pytest.mark.parametrize("G,n,p,intercept,one_launch", [
+    (1025, 43690, 5, 1, True), (1025, 21845, 5, 0, True), (1025, 21846, 5, 0, False),
+    (1024, 37449, 6, 0, True), (1025, 18724, 6, 1, True), (1025, 18725, 6, 1, False),
+    (1025, 8192, 10, 0, True), (1025, 8193, 10, 0, False), (5001, 9362, 6, 1, True),
+    (5001, 9363, 6, 1, False), (20001, 64, 8, 1, True), (20001, 64, 7, 0, True),
+    (5000, 64, 8, 0, True), (5001, 64, 8, 0, False), (5001, 2978, 10, 1, True),
+    (5001, 2979, 10, 1, False), (20000, 64, 9, 1, True), (20001, 64, 9, 1, False)])
+def test_rule_of_the_gene_kernel(dv, G, n, p, intercept, one_launch):
+    """The gene kernel runs the whole IRLS in one launch, the rounds in more:
+    both sides of each line of the rule."""
+    print(f"[case] rule G={G} n={n} p={p} intercept={intercept}", flush=True)
     gen = torch.Generator(device="cuda").manual_seed(n)
     Y = torch.poisson(torch.full((G, n), 2.0, device="cuda"), generator=gen).to(torch.int32)
     X = np.random.default_rng(p).normal(size=(n, p))
-    X[:, 0] = 1.0
+    X[:, 0] = 1.0 if intercept else X[:, 0] + 3.0
     ctx = dv.context(0)
     ctx.set_timing(True)
     try:
-        dv.fit_devil(Y, X, overdispersion=False)
+        dv.fit_devil(Y, X, overdispersion=False, max_iter=3)
         launches = ctx.kernel_stats()["irls_fp64"][0]
     finally:
         ctx.set_timing(False)
