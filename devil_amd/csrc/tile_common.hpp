@@ -191,9 +191,11 @@ __device__ __forceinline__ void load_tile_tables(const TileDesign& td, int64_t b
 // last 16-column tile is time: 4 instructions of 64 cycles per block.  With at
 // most kMaxVCols columns in it they are summed by vector instructions instead,
 // 4 per column and block (VC of them compiled in).  IRLS of 4000 genes x
-// 500000 cells, p = 8 (33 columns): 65.7 -> 57.9 ms; with four columns (1500 x
-// 310683, p = 6: 20) their operands cost the third wave of a SIMD, 13.2 ->
-// 13.9 ms, so three and four stay on a matrix tile.
+// 500000 cells, p = 8 (33 columns): 65.7 -> 57.9 ms.  Three and four stay on a
+// matrix tile, where vector instructions are slower: three of 19 columns (1500 x
+// 300000, p = 5) 8.88 -> 9.00 ms, three alone (p = 2) 6.3 -> 7.1; four of 20
+// (1500 x 310683, p = 6), whose operands cost the third wave of a SIMD, 13.2 ->
+// 13.9 ms.
 constexpr int kMaxVCols = 2;
 
 __host__ __device__ inline int vcols_of(int ncol) {
